@@ -373,8 +373,9 @@ void xp_ssd_phase_stats(ssd_t* s, double* busy_s, double* queue_s, double* read_
 int xp_quant_tokens(const uint16_t* x, int64_t T, int64_t H, uint8_t* xq,
                     float* xs, void* stream);
 
-/* Size of route's tile lists for `npairs` pairs over `slots` slots: size
- * `tiles` as 1 + 2 * xp_moe_max_tiles(npairs, slots) ints. */
+/* Size of route's tile lists (and of the scratch its launches share after
+ * them) for `npairs` pairs over `slots` slots: size `tiles` as
+ * 1 + 2 * xp_moe_max_tiles(npairs, slots) ints. */
 int64_t xp_moe_max_tiles(int64_t npairs, int64_t slots);
 
 /* List the pairs whose expert e (0 <= e < num_experts) has
@@ -390,8 +391,9 @@ int xp_moe_route(const void* topk_ids, int topk_elem_bytes, int64_t T,
                  int64_t slots, int32_t* offsets, int32_t* pairs,
                  int32_t* tiles, void* stream);
 
-/* xp_quant_tokens and xp_moe_route in one launch (the decode step's
- * quantisation and routing). Same arguments and results as the two calls. */
+/* xp_quant_tokens and xp_moe_route in one launch up to 4096 pairs (the
+ * decode step's quantisation and routing), two above. Same arguments and
+ * results as the two calls. */
 int xp_moe_quant_route(const uint16_t* x, int64_t T, int64_t H, uint8_t* xq,
                        float* xs, const void* topk_ids, int topk_elem_bytes,
                        int64_t topk, const int32_t* expert_map,
@@ -484,6 +486,23 @@ int xp_moe_decode_experts(const uint16_t* x, int64_t T, int64_t H,
 int xp_moe_topk_sum(const uint16_t* contrib, int64_t T, int64_t topk,
                     int64_t H, const void* topk_ids, int topk_elem_bytes,
                     int64_t num_experts, uint16_t* out, void* stream);
+
+/* One MoE layer over a slab: xp_moe_quant_route, xp_moe_experts and
+ * xp_moe_topk_sum in one call, same bits, with everything they hand one
+ * another in `work` (xp_moe_layer_bytes bytes, 256-byte aligned, no initial
+ * contents). expert_map (nullable: expert e has slot e) has num_experts
+ * entries. Pairs whose id is outside [0, num_experts) or whose expert has no
+ * slot below `slots` add nothing. T is at most 65535; the limits of
+ * xp_moe_experts hold. */
+int64_t xp_moe_layer_bytes(int64_t T, int64_t topk, int64_t H, int64_t I,
+                           int64_t slots);
+int xp_moe_layer(const uint16_t* x, int64_t T, int64_t H, const void* topk_ids,
+                 int topk_elem_bytes, int64_t topk, const float* topk_weight,
+                 const int32_t* expert_map, int64_t num_experts, int64_t I,
+                 const uint8_t* w13, const float* w13_scale, const uint8_t* w2,
+                 const float* w2_scale, int64_t slots, void* work,
+                 int64_t work_bytes, uint16_t* out, int activation,
+                 void* stream);
 
 /* ---- measurement ---- */
 

@@ -435,3 +435,65 @@ def test_decode_experts_limits():
     assert not moe.decode_pays(x[:1], ids[:1], 8192)
     assert not moe.decode_fits(x[:1], ids[:1], 8192)  # topk * I above 32 KiB
     assert not moe.decode_fits(torch.zeros((1, 8192), dtype=torch.bfloat16, device="cuda"), ids[:1], 512)
+
+
+# One workgroup routes up to 4096 pairs and several, of at least 1024 pairs
+# each and 64 at most, above: both sides of that line, ragged ranges, a range
+# of more than one batch of 4096 pairs per workgroup (300k pairs), a slot
+# per thread (1024), and a slot that holds every pair.
+@pytest.mark.parametrize("idbits", [32, 64])
+@pytest.mark.parametrize("T, topk, E, slots", [(512, 8, 64, 64), (4097, 1, 20, 12), (683, 6, 300, 256),
+                                               (1024, 8, 2000, 1024), (37500, 8, 256, 256), (5000, 1, 1, 1)])
+def test_route_across_workgroups(T, topk, E, slots, idbits):
+    moe = _moe()
+    g = torch.Generator(device="cuda").manual_seed(T)
+    ids = torch.randint(-1, E + 1, (T, topk), generator=g, device="cuda")
+    emap = torch.randperm(E, generator=g, device="cuda").to(torch.int32) - max(0, min(3, E - slots))
+    r = moe.route(ids.to(torch.int32 if idbits == 32 else torch.int64), emap, slots)
+    flat = ids.flatten()
+    known = (flat >= 0) & (flat < E)
+    slot = torch.where(known, emap[flat.clamp(0, E - 1)].long(), -1)
+    slot = torch.where(slot < slots, slot, -1)
+    count = torch.bincount(slot[slot >= 0], minlength=slots)
+    offsets = r.offsets.long()
+    assert torch.equal(offsets[1:] - offsets[:-1], count) and int(offsets[0]) == 0
+    total = int(offsets[-1])
+    listed = r.pairs[:total].long()
+    assert torch.equal(slot[listed], torch.repeat_interleave(torch.arange(slots, device="cuda"), count))
+    assert torch.equal(listed.sort().values, (slot >= 0).nonzero().flatten())
+    tiles = r.tiles.long().cpu()
+    for at, size, width in ((0, 64, 2), (1 + 2 * _tile_bound(T * topk, slots), 128, 3)):
+        want = [(s, int(offsets[s]) + i, min(size, c - i)) for s, c in enumerate(count.tolist())
+                for i in range(0, c, size)]
+        assert int(tiles[at]) == len(want)
+        got = tiles[at + 1 : at + 1 + width * len(want)].view(-1, width)
+        assert got.tolist() == [list(w[:width]) for w in want]
+
+
+# fused_moe in one native call against the separate public calls, bit for
+# bit: with and without a map, experts without a slot, ids outside the range,
+# fewer experts than the map or the slab has, both id types, one workgroup
+# routing and several.
+@pytest.mark.parametrize("T, topk, E, S, mapped, num", [
+    (1, 4, 16, 16, False, None), (33, 4, 24, 12, True, None), (70, 4, 24, 24, False, 20), (70, 4, 24, 24, False, 30),
+    (700, 6, 40, 40, True, 33), (1100, 4, 64, 64, False, None)])
+@pytest.mark.parametrize("idbits", [32, 64])
+def test_fused_moe_equals_separate_calls(T, topk, E, S, mapped, num, idbits):
+    moe = _moe()
+    H, I = 256, 128
+    x, tw, ids, w13, w13s, w2, w2s = _case(T, S, H, I, T, topk)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    xb, (tw_t, *w) = _bf16(x), _dev(tw, w13, w13s, w2, w2s)
+    ids_t = torch.randint(-2, E + 8, (T, topk), generator=g, device="cuda")
+    ids_t = ids_t.to(torch.int32 if idbits == 32 else torch.int64)
+    emap = torch.randperm(E, generator=g, device="cuda").to(torch.int32) - 2 if mapped else None
+    out = moe.fused_moe(xb, tw_t, ids_t, *w, expert_map=emap, num_experts=num)
+    n = num if num is not None else (E if mapped else S)
+    full = emap if mapped else torch.arange(n, dtype=torch.int32, device="cuda")
+    xq, xs = moe.quant_tokens(xb)
+    contrib = torch.zeros((T * topk, H), dtype=torch.bfloat16, device="cuda")
+    moe.run_experts(xq, xs, tw_t, *w, moe.route(ids_t, full, S), contrib)
+    assert torch.equal(out, moe.topk_sum(contrib, ids_t, n))
+    # The same ids as strided views and weights in another type.
+    wide = torch.stack([ids_t, ids_t], dim=2)[:, :, 0]
+    assert torch.equal(moe.fused_moe(xb, tw_t.double(), wide, *w, expert_map=emap, num_experts=num), out)

@@ -203,24 +203,28 @@ __device__ __forceinline__ int3 block_scan3(int3 v, int3* s_tot, int3* total) {
 // Each wave counts a contiguous range of pairs into its own LDS histogram (no
 // contention between waves), so a slot's list is ordered by wave range;
 // dynamic LDS = 16 * slots ints.
-// Slots of the pairs p0, p0 + 64, ... (kRouteBatch of them; -1 for pairs
-// at or past hi, unknown experts and experts without a slot). All id loads
-// are issued before the first expert_map load, and all of those before any
-// is used, so a batch costs two memory round trips rather than two per pair.
-constexpr int kRouteBatch = 16;
+constexpr int64_t kRouteOne = 4096;  // pairs up to which one workgroup routes
+constexpr int kRouteBatch = kRouteOne / kRouteThreads;
+
+// Slots of the pairs p0, p0 + STRIDE, ... (N of them; -1 for pairs at or past
+// hi, unknown experts and experts without a slot; without a map, expert e
+// has slot e). All id loads are issued before the first expert_map load, and
+// all of those before any is used: two memory round trips in all rather than
+// two per pair.
+template <int N, int STRIDE>
 __device__ __forceinline__ void route_slots(const void* ids, int eb, int64_t p0, int64_t hi,
-                                            const int32_t* __restrict__ expert_map, int E, int slots,
-                                            int (&sl)[kRouteBatch]) {
-  int64_t e[kRouteBatch];
+                                            const int32_t* __restrict__ expert_map, int E, int slots, int (&sl)[N]) {
+  int64_t e[N];
 #pragma unroll
-  for (int j = 0; j < kRouteBatch; ++j) {
-    const int64_t p = p0 + 64 * j;
+  for (int j = 0; j < N; ++j) {
+    const int64_t p = p0 + STRIDE * j;
     e[j] = p < hi ? load_id(ids, eb, p) : -1;
   }
 #pragma unroll
-  for (int j = 0; j < kRouteBatch; ++j) sl[j] = (e[j] >= 0 && e[j] < E) ? expert_map[e[j]] : -1;
+  for (int j = 0; j < N; ++j)
+    sl[j] = (e[j] >= 0 && e[j] < E) ? (expert_map ? expert_map[e[j]] : static_cast<int>(e[j])) : -1;
 #pragma unroll
-  for (int j = 0; j < kRouteBatch; ++j) sl[j] = sl[j] < slots ? sl[j] : -1;
+  for (int j = 0; j < N; ++j) sl[j] = sl[j] < slots ? sl[j] : -1;
 }
 
 __device__ __forceinline__ void route_block(const void* ids, int eb, int64_t npairs,
@@ -235,25 +239,12 @@ __device__ __forceinline__ void route_block(const void* ids, int eb, int64_t npa
   const int64_t per = (npairs + kW - 1) / kW;
   const int64_t lo = wave * per, hi = lo + per < npairs ? lo + per : npairs;
   int* hist = s_hist + wave * slots;
-  // A wave whose range is one batch (up to 16384 pairs in all) keeps its
-  // slots in registers for the scatter below instead of loading the ids and
-  // expert_map again (two memory round trips).
-  const bool one = hi - lo <= 64 * kRouteBatch;
-  int sl1[kRouteBatch];
-  if (one) {
-    route_slots(ids, eb, lo + lane, hi, expert_map, E, slots, sl1);
+  // A wave's range is at most one batch, kept in registers for the scatter.
+  int sl[kRouteBatch];
+  route_slots<kRouteBatch, 64>(ids, eb, lo + lane, hi, expert_map, E, slots, sl);
 #pragma unroll
-    for (int j = 0; j < kRouteBatch; ++j)
-      if (sl1[j] >= 0) atomicAdd(&hist[sl1[j]], 1);
-  } else {
-    for (int64_t b = lo; b < hi; b += 64 * kRouteBatch) {
-      int sl[kRouteBatch];
-      route_slots(ids, eb, b + lane, hi, expert_map, E, slots, sl);
-#pragma unroll
-      for (int j = 0; j < kRouteBatch; ++j)
-        if (sl[j] >= 0) atomicAdd(&hist[sl[j]], 1);
-    }
-  }
+  for (int j = 0; j < kRouteBatch; ++j)
+    if (sl[j] >= 0) atomicAdd(&hist[sl[j]], 1);
   __syncthreads();
   int c = 0;
   if (tid < slots) {
@@ -286,19 +277,9 @@ __device__ __forceinline__ void route_block(const void* ids, int eb, int64_t npa
     if (wide) wide[0] = total.z;
   }
   __syncthreads();
-  if (one) {
 #pragma unroll
-    for (int j = 0; j < kRouteBatch; ++j)
-      if (sl1[j] >= 0) pairs[atomicAdd(&hist[sl1[j]], 1)] = static_cast<int32_t>(lo + lane + 64 * j);
-    return;
-  }
-  for (int64_t b = lo; b < hi; b += 64 * kRouteBatch) {
-    int sl[kRouteBatch];
-    route_slots(ids, eb, b + lane, hi, expert_map, E, slots, sl);
-#pragma unroll
-    for (int j = 0; j < kRouteBatch; ++j)
-      if (sl[j] >= 0) pairs[atomicAdd(&hist[sl[j]], 1)] = static_cast<int32_t>(b + lane + 64 * j);
-  }
+  for (int j = 0; j < kRouteBatch; ++j)
+    if (sl[j] >= 0) pairs[atomicAdd(&hist[sl[j]], 1)] = static_cast<int32_t>(lo + lane + 64 * j);
 }
 
 __global__ void __launch_bounds__(kRouteThreads) route_kernel(const void* ids, int eb, int64_t npairs,
@@ -331,6 +312,120 @@ __global__ void __launch_bounds__(kRouteThreads) quant_route_kernel(const uint16
   }
   const int64_t t = (static_cast<int64_t>(blockIdx.x) - 1) * 4 + (threadIdx.x >> 8);
   if (t < T) quant_token(x, H, xq, xs, t, threadIdx.x & 255);
+}
+
+// ---- routing of many pairs: counted and scattered by several workgroups ----
+//
+// One workgroup is bound by its own LDS atomics and load round trips (two
+// atomics a pair): 17 us at 16384 pairs over 256 slots, 81 us at 65536.
+// Above kRouteOne pairs, `nb` workgroups each count a contiguous range of
+// pairs into LDS and write their slot counts to the scratch after the wide
+// list, beside the token quantisation where the call has one; a second
+// launch of nb workgroups sums those counts (every workgroup for itself:
+// nb x slots ints out of L2), scans them, and scatters its own range.
+// 65536 pairs with 8192 tokens to quantise: 81 + 15 -> 19 + 9 us; 16384 with
+// 2048: 17 + 5 -> 6 + 5 us. At 2664 pairs one workgroup takes 6 us beside the
+// quantisation, as long as the two launches, so it keeps the small calls.
+constexpr int64_t kRouteRange = 1024;   // pairs per workgroup, at least
+constexpr int kRouteBlocks = 64;        // workgroups at most
+constexpr int kCountBatch = 4;          // pairs a thread keeps in flight
+
+// Workgroups that route npairs pairs (0: one workgroup, no count launch).
+__host__ __device__ inline int route_blocks(int64_t npairs) {
+  if (npairs <= kRouteOne) return 0;
+  const int64_t nb = (npairs + kRouteRange - 1) / kRouteRange;
+  return static_cast<int>(nb < kRouteBlocks ? nb : kRouteBlocks);
+}
+
+// Workgroups 0 .. nb - 1: hist[b][slots] = pairs of each slot in range b.
+// The others quantise four tokens each (x null: none).
+__global__ void __launch_bounds__(kRouteThreads) quant_count_kernel(const uint16_t* __restrict__ x, int64_t T,
+                                                                    int64_t H, uint8_t* __restrict__ xq,
+                                                                    float* __restrict__ xs, const void* ids, int eb,
+                                                                    int64_t npairs, int nb,
+                                                                    const int32_t* __restrict__ expert_map, int E,
+                                                                    int slots, int32_t* __restrict__ hist) {
+  __shared__ int s_count[kMaxRouteSlots];
+  const int tid = threadIdx.x, b = blockIdx.x;
+  if (b >= nb) {
+    const int64_t t = (static_cast<int64_t>(b) - nb) * 4 + (tid >> 8);
+    if (t < T) quant_token(x, H, xq, xs, t, tid & 255);
+    return;
+  }
+  const int64_t per = (npairs + nb - 1) / nb;
+  const int64_t lo = b * per, hi = lo + per < npairs ? lo + per : npairs;
+  s_count[tid] = 0;
+  __syncthreads();
+  for (int64_t p = lo + tid; p < hi; p += kRouteThreads * kCountBatch) {
+    int sl[kCountBatch];
+    route_slots<kCountBatch, kRouteThreads>(ids, eb, p, hi, expert_map, E, slots, sl);
+#pragma unroll
+    for (int j = 0; j < kCountBatch; ++j)
+      if (sl[j] >= 0) atomicAdd(&s_count[sl[j]], 1);
+  }
+  __syncthreads();
+  if (tid < slots) hist[static_cast<int64_t>(b) * slots + tid] = s_count[tid];
+}
+
+// route_kernel's results from the counts, by nb = gridDim.x workgroups;
+// workgroup 0 writes offsets and tiles, the last one the wide tiles.
+__global__ void __launch_bounds__(kRouteThreads) route_scatter_kernel(
+    const void* ids, int eb, int64_t npairs, const int32_t* __restrict__ expert_map, int E, int slots,
+    const int32_t* __restrict__ hist, int32_t* __restrict__ offsets, int32_t* __restrict__ pairs,
+    int32_t* __restrict__ tiles, int32_t* __restrict__ wide) {
+  __shared__ int s_cur[kMaxRouteSlots];
+  __shared__ int3 s_tot[kRouteThreads / 64];
+  const int tid = threadIdx.x, b = blockIdx.x, nb = gridDim.x;
+  const int64_t per = (npairs + nb - 1) / nb;
+  const int64_t lo = b * per, hi = lo + per < npairs ? lo + per : npairs;
+  int first[kCountBatch];  // the first pairs' slots, requested before the counts
+  route_slots<kCountBatch, kRouteThreads>(ids, eb, lo + tid, hi, expert_map, E, slots, first);
+  int c = 0, before = 0;
+  if (tid < slots) {
+#pragma unroll 8
+    for (int i = 0; i < nb; ++i) {
+      const int v = hist[static_cast<int64_t>(i) * slots + tid];
+      c += v;
+      before += i < b ? v : 0;
+    }
+  }
+  const int nt = (c + kBM - 1) / kBM, nw = (c + kWM - 1) / kWM;
+  int3 total;
+  const int3 off = block_scan3(make_int3(c, nt, nw), s_tot, &total);
+  if (tid < slots) {
+    s_cur[tid] = off.x + before;
+    if (b == 0) {
+      offsets[tid] = off.x;
+      for (int i = 0; i < nt; ++i) {
+        tiles[1 + 2 * (off.y + i)] = tid;
+        tiles[2 + 2 * (off.y + i)] = off.x + i * kBM;
+      }
+    }
+    if (b == nb - 1)
+      for (int i = 0; i < nw; ++i) {
+        wide[1 + 3 * (off.z + i)] = tid;
+        wide[2 + 3 * (off.z + i)] = off.x + i * kWM;
+        wide[3 + 3 * (off.z + i)] = c - i * kWM < kWM ? c - i * kWM : kWM;
+      }
+  }
+  if (tid == 0 && b == 0) {
+    offsets[slots] = total.x;
+    tiles[0] = total.y;
+  }
+  if (tid == 0 && b == nb - 1) wide[0] = total.z;
+  __syncthreads();
+  for (int64_t p = lo + tid; p < hi; p += kRouteThreads * kCountBatch) {
+    int sl[kCountBatch];
+    if (p == lo + tid) {
+#pragma unroll
+      for (int j = 0; j < kCountBatch; ++j) sl[j] = first[j];
+    } else {
+      route_slots<kCountBatch, kRouteThreads>(ids, eb, p, hi, expert_map, E, slots, sl);
+    }
+#pragma unroll
+    for (int j = 0; j < kCountBatch; ++j)
+      if (sl[j] >= 0) pairs[atomicAdd(&s_cur[sl[j]], 1)] = static_cast<int32_t>(p + kRouteThreads * j);
+  }
 }
 
 struct Tile {
@@ -376,6 +471,12 @@ __host__ __device__ inline int64_t wide_bound(int64_t npairs, int64_t slots) {
 // pair count) per wide tile.
 __host__ __device__ inline int64_t wide_list_offset(int64_t npairs, int64_t slots) {
   return 1 + 2 * tile_bound(npairs, slots);
+}
+
+// The counts of the routing workgroups, after the wide list's 1 + 3 *
+// wide_bound ints: [workgroup][slot].
+__host__ __device__ inline int64_t route_hist_offset(int64_t npairs, int64_t slots) {
+  return wide_list_offset(npairs, slots) + 1 + 3 * wide_bound(npairs, slots);
 }
 
 // Workspace of xp_moe_experts: bf16 activations, their per-16-column
@@ -1870,10 +1971,13 @@ __global__ void __launch_bounds__(kGemmWaves * 64) gemm2_kernel(int64_t H, int64
 }
 
 // out[t] = bf16(sum over k of contrib[t*topk + k]) in fp32, k ascending,
-// over the pairs whose id is a valid expert.
+// over the pairs whose id is a valid expert and, given a map, whose expert
+// has a slot (the contribution of one without was never written).
 template <typename Id>
 __global__ void __launch_bounds__(256) topk_sum_kernel(const uint16_t* __restrict__ contrib, int64_t H, int topk,
-                                                       const Id* __restrict__ ids, int E, uint16_t* __restrict__ out) {
+                                                       const Id* __restrict__ ids, int E,
+                                                       const int32_t* __restrict__ expert_map, int slots,
+                                                       uint16_t* __restrict__ out) {
   const int64_t t = blockIdx.y;
   const int64_t c = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 8;
   if (c >= H) return;
@@ -1890,6 +1994,10 @@ __global__ void __launch_bounds__(256) topk_sum_kernel(const uint16_t* __restric
       const int64_t p = t * topk + k;
       const int64_t e = ids[p];
       ok[i] = k0 + i < topk && e >= 0 && e < E;
+      if (expert_map && ok[i]) {
+        const int sl = expert_map[e];
+        ok[i] = sl >= 0 && sl < slots;
+      }
       v[i] = *reinterpret_cast<const u32x4*>(contrib + p * H + c);
     }
 #pragma unroll
@@ -1908,6 +2016,35 @@ __global__ void __launch_bounds__(256) topk_sum_kernel(const uint16_t* __restric
   *reinterpret_cast<u32x4*>(out + t * H + c) = o;
 }
 
+// Routing of npairs pairs, with the quantisation of T tokens where x is given.
+int launch_route(const uint16_t* x, int64_t T, int64_t H, uint8_t* xq, float* xs, const void* ids, int eb,
+                 int64_t npairs, const int32_t* expert_map, int64_t num_experts, int64_t slots, int32_t* offsets,
+                 int32_t* pairs, int32_t* tiles, void* stream) {
+  const hipStream_t st = as_stream(stream);
+  const int E = static_cast<int>(num_experts), S = static_cast<int>(slots);
+  int32_t* wide = npairs > 0 ? tiles + wide_list_offset(npairs, slots) : nullptr;
+  const int64_t quant_blocks = x ? (T + 3) / 4 : 0;
+  const int nb = route_blocks(npairs);
+  if (nb > 0) {
+    int32_t* hist = tiles + route_hist_offset(npairs, slots);
+    hipLaunchKernelGGL(quant_count_kernel, dim3(static_cast<unsigned>(nb + quant_blocks)), dim3(kRouteThreads), 0, st,
+                       x, x ? T : 0, H, xq, xs, ids, eb, npairs, nb, expert_map, E, S, hist);
+    if (int rc = check_launch("quant_count_kernel")) return rc;
+    hipLaunchKernelGGL(route_scatter_kernel, dim3(static_cast<unsigned>(nb)), dim3(kRouteThreads), 0, st, ids, eb,
+                       npairs, expert_map, E, S, hist, offsets, pairs, tiles, wide);
+    return check_launch("route_scatter_kernel");
+  }
+  const size_t lds = static_cast<size_t>(kRouteThreads / 64) * static_cast<size_t>(slots) * sizeof(int);
+  if (x) {
+    hipLaunchKernelGGL(quant_route_kernel, dim3(static_cast<unsigned>(1 + quant_blocks)), dim3(kRouteThreads), lds,
+                       st, x, T, H, xq, xs, ids, eb, npairs, expert_map, E, S, offsets, pairs, tiles, wide);
+    return check_launch("quant_route_kernel");
+  }
+  hipLaunchKernelGGL(route_kernel, dim3(1), dim3(kRouteThreads), lds, st, ids, eb, npairs, expert_map, E, S, offsets,
+                     pairs, tiles, wide);
+  return check_launch("route_kernel");
+}
+
 }  // namespace
 }  // namespace xp
 
@@ -1917,9 +2054,10 @@ extern "C" {
 
 int64_t xp_moe_max_tiles(int64_t npairs, int64_t slots) {
   if (npairs <= 0 || slots <= 0) return 0;
-  // The tile list, then the wide-tile list (1 + 3 * wide_bound ints), in
-  // two-int entries past tiles[0].
-  return tile_bound(npairs, slots) + (2 + 3 * wide_bound(npairs, slots)) / 2;
+  // The tile list, then the wide-tile list (1 + 3 * wide_bound ints) and the
+  // routing workgroups' counts, in two-int entries past tiles[0].
+  const int64_t ints = route_hist_offset(npairs, slots) - 1 + route_blocks(npairs) * slots;
+  return (ints + 1) / 2;
 }
 
 int xp_quant_tokens(const uint16_t* x, int64_t T, int64_t H, uint8_t* xq, float* xs, void* stream) {
@@ -1942,12 +2080,8 @@ int xp_moe_route(const void* topk_ids, int topk_elem_bytes, int64_t T, int64_t t
              kMaxRouteSlots);
   XP_REQUIRE(num_experts >= 1 && num_experts <= INT32_MAX, "xp_moe_route: %lld experts", (long long)num_experts);
   XP_REQUIRE(expert_map && offsets && pairs && tiles && (T == 0 || topk_ids), "xp_moe_route: null argument");
-  const size_t lds = static_cast<size_t>(kRouteThreads / 64) * static_cast<size_t>(slots) * sizeof(int);
-  int32_t* wide = T * topk > 0 ? tiles + wide_list_offset(T * topk, slots) : nullptr;
-  hipLaunchKernelGGL(route_kernel, dim3(1), dim3(kRouteThreads), lds, as_stream(stream), topk_ids, topk_elem_bytes,
-                     T * topk, expert_map, static_cast<int>(num_experts), static_cast<int>(slots), offsets, pairs,
-                     tiles, wide);
-  return check_launch("route_kernel");
+  return launch_route(nullptr, 0, 0, nullptr, nullptr, topk_ids, topk_elem_bytes, T * topk, expert_map, num_experts,
+                      slots, offsets, pairs, tiles, stream);
 }
 
 int xp_moe_quant_route(const uint16_t* x, int64_t T, int64_t H, uint8_t* xq, float* xs, const void* topk_ids,
@@ -1965,13 +2099,8 @@ int xp_moe_quant_route(const uint16_t* x, int64_t T, int64_t H, uint8_t* xq, flo
   XP_REQUIRE(expert_map && offsets && pairs && tiles, "xp_moe_quant_route: null argument");
   XP_REQUIRE(T == 0 || (x && xq && xs && topk_ids && aligned16(x) && aligned16(xq)),
              "xp_moe_quant_route: null or misaligned buffer");
-  const size_t lds = static_cast<size_t>(kRouteThreads / 64) * static_cast<size_t>(slots) * sizeof(int);
-  const unsigned grid = static_cast<unsigned>(1 + (T + 3) / 4);
-  int32_t* wide = T * topk > 0 ? tiles + wide_list_offset(T * topk, slots) : nullptr;
-  hipLaunchKernelGGL(quant_route_kernel, dim3(grid), dim3(kRouteThreads), lds, as_stream(stream), x, T, H, xq, xs,
-                     topk_ids, topk_elem_bytes, T * topk, expert_map, static_cast<int>(num_experts),
-                     static_cast<int>(slots), offsets, pairs, tiles, wide);
-  return check_launch("quant_route_kernel");
+  return launch_route(x, T, H, xq, xs, topk_ids, topk_elem_bytes, T * topk, expert_map, num_experts, slots, offsets,
+                      pairs, tiles, stream);
 }
 
 int64_t xp_moe_workspace_bytes(int64_t npairs, int64_t I) {
@@ -2107,10 +2236,94 @@ int launch_experts(const uint8_t* xq, const float* xs, int64_t T, int64_t topk, 
   return check_launch("gemm2_narrow_kernel");
 }
 
+int launch_topk_sum(const uint16_t* contrib, int64_t T, int64_t topk, int64_t H, const void* ids, int eb,
+                    int64_t num_experts, const int32_t* expert_map, int64_t slots, uint16_t* out, void* stream) {
+  const dim3 grid(static_cast<unsigned>((H / 8 + 255) / 256), static_cast<unsigned>(T));
+  if (eb == 8)
+    hipLaunchKernelGGL(topk_sum_kernel<int64_t>, grid, dim3(256), 0, as_stream(stream), contrib, H,
+                       static_cast<int>(topk), static_cast<const int64_t*>(ids), static_cast<int>(num_experts),
+                       expert_map, static_cast<int>(slots), out);
+  else
+    hipLaunchKernelGGL(topk_sum_kernel<int32_t>, grid, dim3(256), 0, as_stream(stream), contrib, H,
+                       static_cast<int>(topk), static_cast<const int32_t*>(ids), static_cast<int>(num_experts),
+                       expert_map, static_cast<int>(slots), out);
+  return check_launch("topk_sum_kernel");
+}
+
+// Workspace of xp_moe_layer: what the separate calls hand one another, then
+// xp_moe_experts' workspace.
+struct LayerWork {
+  uint8_t* xq;        // [T][H]
+  float* xs;          // [T][H/128]
+  int32_t* offsets;   // [slots + 1]
+  int32_t* pairs;     // [T * topk]
+  int32_t* tiles;     // [1 + 2 * max_tiles]
+  uint16_t* contrib;  // [T * topk][H]
+  uint8_t* ffn;
+};
+
+int64_t layer_layout(int64_t T, int64_t topk, int64_t H, int64_t I, int64_t slots, LayerWork* w, uint8_t* base) {
+  const int64_t n = T * topk;
+  const int64_t sz[7] = {align256(T * H),
+                         align256(T * (H / kKB) * 4),
+                         align256((slots + 1) * 4),
+                         align256(n * 4),
+                         align256((1 + 2 * xp_moe_max_tiles(n, slots)) * 4),
+                         align256(n * H * 2),
+                         work_layout(n, I, nullptr, nullptr)};
+  int64_t at[8] = {0};
+  for (int i = 0; i < 7; ++i) at[i + 1] = at[i] + sz[i];
+  if (w) {
+    w->xq = base;
+    w->xs = reinterpret_cast<float*>(base + at[1]);
+    w->offsets = reinterpret_cast<int32_t*>(base + at[2]);
+    w->pairs = reinterpret_cast<int32_t*>(base + at[3]);
+    w->tiles = reinterpret_cast<int32_t*>(base + at[4]);
+    w->contrib = reinterpret_cast<uint16_t*>(base + at[5]);
+    w->ffn = base + at[6];
+  }
+  return at[7];
+}
+
 }  // namespace
 }  // namespace xp
 
 extern "C" {
+
+int64_t xp_moe_layer_bytes(int64_t T, int64_t topk, int64_t H, int64_t I, int64_t slots) {
+  if (T <= 0 || topk <= 0 || H <= 0 || I <= 0 || slots <= 0) return 0;
+  return layer_layout(T, topk, H, I, slots, nullptr, nullptr);
+}
+
+int xp_moe_layer(const uint16_t* x, int64_t T, int64_t H, const void* topk_ids, int topk_elem_bytes, int64_t topk,
+                 const float* topk_weight, const int32_t* expert_map, int64_t num_experts, int64_t I,
+                 const uint8_t* w13, const float* w13_scale, const uint8_t* w2, const float* w2_scale, int64_t slots,
+                 void* work, int64_t work_bytes, uint16_t* out, int activation, void* stream) {
+  const char* what = "xp_moe_layer";
+  XP_REQUIRE(activation == XP_ACT_SILU || activation == XP_ACT_GELU, "%s: unknown activation %d", what, activation);
+  XP_REQUIRE(topk_elem_bytes == 4 || topk_elem_bytes == 8, "%s: id size %d", what, topk_elem_bytes);
+  XP_REQUIRE(num_experts >= 1 && num_experts <= INT32_MAX, "%s: %lld experts", what, (long long)num_experts);
+  XP_REQUIRE(T >= 0 && T <= 65535, "%s: T=%lld (at most 65535)", what, (long long)T);
+  XP_REQUIRE(T == 0 || (work && (reinterpret_cast<uintptr_t>(work) & 255) == 0),
+             "%s: the workspace must be non-null and 256-byte aligned", what);
+  LayerWork w{};
+  const int64_t need = xp_moe_layer_bytes(T, topk, H, I, slots);
+  if (T > 0) layer_layout(T, topk, H, I, slots, &w, static_cast<uint8_t*>(work));
+  int rc = check_ffn(what, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots, w.offsets, w.pairs,
+                     w.tiles, out);
+  if (rc || T == 0) return rc;
+  XP_REQUIRE(work_bytes >= need, "%s: workspace of %lld B, needs %lld", what, (long long)work_bytes, (long long)need);
+  XP_REQUIRE(x && topk_ids && aligned16(x), "%s: x and topk_ids must be non-null, x 16-byte aligned", what);
+  rc = launch_route(x, T, H, w.xq, w.xs, topk_ids, topk_elem_bytes, T * topk, expert_map, num_experts, slots,
+                    w.offsets, w.pairs, w.tiles, stream);
+  if (rc) return rc;
+  rc = launch_experts(w.xq, w.xs, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots, w.offsets,
+                      w.pairs, w.tiles, w.ffn, w.contrib, activation, stream);
+  if (rc) return rc;
+  // Without a map expert e has slot e, so the sum's bound on the ids says it all.
+  const int64_t E = expert_map || num_experts < slots ? num_experts : slots;
+  return launch_topk_sum(w.contrib, T, topk, H, topk_ids, topk_elem_bytes, E, expert_map, slots, out, stream);
+}
 
 int xp_moe_experts(const uint8_t* xq, const float* xs, int64_t T, int64_t topk, const float* topk_weight, int64_t H,
                    int64_t I, const uint8_t* w13, const float* w13_scale, const uint8_t* w2, const float* w2_scale,
@@ -2213,16 +2426,7 @@ int xp_moe_topk_sum(const uint16_t* contrib, int64_t T, int64_t topk, int64_t H,
   if (T == 0) return XP_OK;
   XP_REQUIRE(contrib && out && topk_ids && aligned16(contrib) && aligned16(out),
              "xp_moe_topk_sum: null or misaligned buffer");
-  const unsigned bx = static_cast<unsigned>((H / 8 + 255) / 256);
-  if (topk_elem_bytes == 8)
-    hipLaunchKernelGGL(topk_sum_kernel<int64_t>, dim3(bx, static_cast<unsigned>(T)), dim3(256), 0, as_stream(stream),
-                       contrib, H, static_cast<int>(topk), static_cast<const int64_t*>(topk_ids),
-                       static_cast<int>(num_experts), out);
-  else
-    hipLaunchKernelGGL(topk_sum_kernel<int32_t>, dim3(bx, static_cast<unsigned>(T)), dim3(256), 0, as_stream(stream),
-                       contrib, H, static_cast<int>(topk), static_cast<const int32_t*>(topk_ids),
-                       static_cast<int>(num_experts), out);
-  return check_launch("topk_sum_kernel");
+  return launch_topk_sum(contrib, T, topk, H, topk_ids, topk_elem_bytes, num_experts, nullptr, 0, out, stream);
 }
 
 }  // extern "C"

@@ -312,6 +312,17 @@ int xp_encode_rows(const uint8_t* raw, int64_t rows, int64_t raw_stride,
                    uint8_t* luts, int64_t lut_stride, int64_t* needed,
                    void* stream);
 
+/* xp_encode_rows with a workspace (xp_encode_workspace_bytes bytes, device
+ * memory, no initial contents), in which several workgroups plan a row: the
+ * faster form for any number of rows, many times so for a few. Same bytes;
+ * a null `work` is xp_encode_rows. */
+int64_t xp_encode_workspace_bytes(int64_t rows, int64_t n, int64_t chunk);
+int xp_encode_rows_split(const uint8_t* raw, int64_t rows, int64_t raw_stride,
+                         int64_t n, int64_t chunk, uint8_t* records,
+                         int64_t pitch, uint8_t* luts, int64_t lut_stride,
+                         int64_t* needed, void* work, int64_t work_bytes,
+                         void* stream);
+
 /* Code of a 16-symbol histogram: lengths[16], bit-reversed codes[16] and
  * lut[512] ((sym << 4) | len). Replaces code_lengths / Code
  * (codec.py:61-114). */

@@ -124,3 +124,37 @@ def test_encode_of_a_gpu_row():
     hrec, hlut, _ = _host(codec, raw, pitch, 512)
     np.testing.assert_array_equal(rec.cpu().numpy(), hrec)
     np.testing.assert_array_equal(lut.cpu().numpy(), hlut)
+
+
+# The plan by several workgroups per row against the one by a workgroup per
+# row: rows of 1, 2, 4 and 8 groups per counting workgroup (up to 2048
+# workgroups take one group each), more than one 64 KiB part per row, and rows
+# that do not fit, whose records stay as they were.
+@pytest.mark.parametrize("count, groups, chunk", [(1, 1, 16), (1, 130, 64), (300, 9, 16), (700, 11, 16),
+                                                  (1500, 17, 16), (3, 40, 1024)])
+def test_split_plan_equals_a_workgroup_per_row(count, groups, chunk):
+    from vllm_expert_pager import _native as nat
+
+    n = groups * chunk * 32
+    g = torch.Generator(device="cuda").manual_seed(n)
+    sharp = torch.rand((count, 1), generator=g, device="cuda") * 6  # from uniform exponents to a few of them
+    raw = (torch.rand((count, n), generator=g, device="cuda") ** (1 + sharp) * 256).to(torch.uint8)
+    # The median row's size: some rows fit and some do not.
+    needed = _codec().encode_rows(raw, codec_ref.pitch_of(n, 1.6, 16), chunk, check=False)[2]
+    pitch = int(needed.median()) // 16 * 16
+    outs = []
+    for name in ("xp_encode_rows", "xp_encode_rows_split"):
+        rec = torch.full((count, pitch), 0x5A, dtype=torch.uint8, device="cuda")
+        lut = torch.zeros((count, 512), dtype=torch.uint8, device="cuda")
+        needed = torch.zeros((count,), dtype=torch.int64, device="cuda")
+        nbytes = nat.lib().xp_encode_workspace_bytes(count, n, chunk)
+        work = torch.empty((nbytes,), dtype=torch.uint8, device="cuda")
+        tail = (work.data_ptr(), nbytes) if name.endswith("split") else ()
+        nat.call(name, raw.data_ptr(), count, n, n, chunk, rec.data_ptr(), pitch, lut.data_ptr(), 512,
+                 needed.data_ptr(), *tail, nat.stream())
+        outs.append((rec, lut, needed))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    over = outs[0][2] > pitch
+    assert bool((outs[0][0][over] == 0x5A).all())
+    assert count < 300 or 0 < int(over.sum()) < count

@@ -1,10 +1,11 @@
 // Batched GPU encoder of the fp8 exponent Huffman row format
 // (encode, codec.py:125-198), producing the bytes of the host encoder
-// (codec_host.cpp) and of the reference. Two launches:
+// (codec_host.cpp) and of the reference.
 //
-// encode_plan_kernel, one workgroup per row:
+// The plan: encode_hist_kernel and encode_words_kernel, several workgroups
+// per row, or without a workspace encode_plan_kernel, one per row:
 //   1. exponent histogram: per-thread counters in LDS, then summed;
-//   2. the code (code_build.h) by one thread, the 512-entry LUT by all;
+//   2. the code by one wave, the 512-entry LUT by the workgroup;
 //   3. Huffman words per chunk: the decoder loads a word before symbol i
 //      whenever fewer than LIMIT bits are left, so a chunk whose last symbol
 //      starts at bit b needs (b + LIMIT - 1) / 32 + 1 words; summed per
@@ -19,9 +20,10 @@
 //      refilling lanes below, as the decoder computes it. A lane emits a
 //      word once its 32 bits are complete; at most two refills are waiting
 //      for their word. The lane also writes its sign/mantissa nibble words.
-// The record is written whole: gstart and the zero tail up to the pitch by
-// the first launch, nibbles and Huffman words by the second. A row that does
-// not fit its pitch writes nothing but its LUT and needed bytes.
+// The record is written whole: nibbles and Huffman words by the groups
+// launch, gstart and the zero tail up to the pitch by it or by
+// encode_plan_kernel. A row that does not fit its pitch writes nothing but its
+// LUT and needed bytes.
 #include "code_build.h"
 #include "common.h"
 
@@ -50,7 +52,100 @@ struct EncodeArgs {
   uint8_t* lut;
   int64_t lut_stride;  // bytes between LUTs
   int64_t* needed;     // record bytes each row needs
+  uint32_t* hist;      // split plan: [row][part][16] exponent counts
+  int32_t* words;      // split plan: [row][G] Huffman words per group
+  int parts;           // split plan: parts of a row's histogram
 };
+
+// A row's code, built by one wave and the same in every lane of it: lane l
+// stands for symbol l & 15, whose count it gives and whose code length and
+// code it gets. The lengths are code::code_lengths', whose selection of the
+// lightest node over (count, id) is a merge of two queues: the symbols sorted
+// by (count, symbol), and the merged nodes, which appear in ascending (count,
+// id) order because counts only grow; on equal counts the symbol goes first,
+// as its id is lower. Queue entries live in lane registers (readlane and
+// writelane at wave-uniform indices), so nothing goes through LDS. One thread
+// selecting over 16 nodes, and a LUT looked up entry by entry, were a large
+// part of the 266 us that the plan of one 2 MiB row took.
+__device__ __forceinline__ double lane_double(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+__device__ __forceinline__ int wave_lengths(double count) {
+  const int lane = threadIdx.x & 63, sym = lane & 15;
+  // Place in the sorted order, then sorted counts and symbols by lane.
+  int rank = 0;
+#pragma unroll
+  for (int t = 0; t < code::kSyms; ++t) {
+    const double c = lane_double(count, t);
+    rank += c < count || (c == count && t < sym) ? 1 : 0;
+  }
+  // Queue ends read as infinity: leaves past lane 15, nodes not yet merged.
+  const int to = 4 * ((lane & ~15) + rank);
+  const int inf_hi = 0x7ff00000;
+  int leaf_lo = __builtin_amdgcn_ds_permute(to, __double2loint(count));
+  int leaf_hi = __builtin_amdgcn_ds_permute(to, __double2hiint(count));
+  const int leaf_bit = __builtin_amdgcn_ds_permute(to, 1 << sym);
+  leaf_lo = lane < code::kSyms ? leaf_lo : 0;
+  leaf_hi = lane < code::kSyms ? leaf_hi : inf_hi;
+  int node_lo = 0, node_hi = inf_hi, node_members = 0;  // merged node i in lane i
+  int length = 0;
+  int leaf = 0, head = 0;
+  auto pair_double = [](int hi, int lo, int at) {
+    return __hiloint2double(__builtin_amdgcn_readlane(hi, at), __builtin_amdgcn_readlane(lo, at));
+  };
+  for (int step = 0; step < code::kSyms - 1; ++step) {
+    // The two lightest of the queues' first two entries each.
+    const double l0 = pair_double(leaf_hi, leaf_lo, leaf), l1 = pair_double(leaf_hi, leaf_lo, leaf + 1);
+    const double n0 = pair_double(node_hi, node_lo, head), n1 = pair_double(node_hi, node_lo, head + 1);
+    const int bl0 = __builtin_amdgcn_readlane(leaf_bit, leaf), bl1 = __builtin_amdgcn_readlane(leaf_bit, leaf + 1);
+    const int bn0 = __builtin_amdgcn_readlane(node_members, head);
+    const int bn1 = __builtin_amdgcn_readlane(node_members, head + 1);
+    const int leaves = __builtin_amdgcn_readfirstlane(l1 <= n0 ? 2 : (n1 < l0 ? 0 : 1));
+    const double sum = (leaves > 0 ? l0 : n1) + (leaves == 2 ? l1 : n0);
+    const int members = (leaves > 0 ? bl0 : bn1) | (leaves == 2 ? bl1 : bn0);
+    leaf += leaves;
+    head += 2 - leaves;
+    length += (members >> sym) & 1;
+    node_lo = lane == step ? __double2loint(sum) : node_lo;
+    node_hi = lane == step ? __double2hiint(sum) : node_hi;
+    node_members = lane == step ? members : node_members;
+  }
+  return length;
+}
+
+__device__ __forceinline__ int wave_code_lengths(uint32_t hist) {
+  double count = static_cast<double>(hist > 1 ? hist : 1);
+  for (int k = 0;; ++k) {
+    if (k > 0) {  // as code::code_lengths: k never passes LIMIT
+      double sum = 0.0;
+#pragma unroll
+      for (int i = 0; i < code::kSyms; ++i) sum += lane_double(count, i);
+      const double floor_c = sum / static_cast<double>(1 << (XP_LIMIT - k));
+      count = count > floor_c ? count : floor_c;
+    }
+    const int length = wave_lengths(count);
+    if (!__builtin_amdgcn_ballot_w64(length > XP_LIMIT)) return length;
+  }
+}
+
+// code::canonical_codes of lane l's symbol l & 15.
+__device__ __forceinline__ int wave_canonical_code(int length) {
+  const int lane = threadIdx.x & 63, sym = lane & 15;
+  uint32_t first = 0, code = 0, prev = 0, below = 0;
+#pragma unroll
+  for (int L = 1; L <= XP_LIMIT; ++L) {
+    const uint32_t of = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(length == L)) & 0xffffu;
+    code = (code + prev) << 1;
+    prev = static_cast<uint32_t>(__popc(of));
+    if (length == L) {
+      first = code;
+      below = static_cast<uint32_t>(__popc(of & ((1u << sym) - 1u)));
+    }
+  }
+  return static_cast<int>(__brev(first + below) >> (32 - length));
+}
 
 // Lengths of the four bytes of w as a sum. lb[k] holds the code lengths of
 // symbols 4k..4k+3 as bytes. Each byte's symbol (its exponent field) selects
@@ -66,6 +161,151 @@ __device__ __forceinline__ uint32_t sum_lengths4(uint32_t w, const uint32_t (&lb
   return __builtin_amdgcn_sad_u8(__builtin_amdgcn_perm(b, a, pick), 0u, 0u);
 }
 
+// The code lengths as bytes, symbol s in byte s % 4 of lb[s / 4].
+__device__ __forceinline__ void pack_lengths(const int32_t* s_len, uint32_t (&lb)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) lb[k] = 0u;
+#pragma unroll
+  for (int s = 0; s < code::kSyms; ++s) lb[s / 4] |= static_cast<uint32_t>(s_len[s]) << (8 * (s % 4));
+}
+
+// Words per chunk: (start bit of its last symbol + LIMIT - 1) / 32 + 1. A
+// thread holds the 16 values at offset off of the row; a chunk's pieces are
+// spread over consecutive threads, so each chunk is summed by a power-of-two
+// set of `per` = chunk / 16 lanes of one wave (at most 64), and its last lane
+// adds the chunk's words to its group's.
+__device__ __forceinline__ void add_chunk_words(const u32x4& v, int64_t off, int chunk, int per,
+                                                const uint32_t (&lb)[4], int32_t* s_words, int64_t g_base) {
+  uint32_t bits = sum_lengths4(v.x, lb) + sum_lengths4(v.y, lb) + sum_lengths4(v.z, lb) + sum_lengths4(v.w, lb);
+  const bool last = ((off + 16) % chunk) == 0;
+  if (last) {  // not the last symbol
+    const uint32_t s3 = v.w >> 27 & 15u;
+    const bool hi = s3 >= 8u;
+    bits -= __builtin_amdgcn_perm(hi ? lb[3] : lb[1], hi ? lb[2] : lb[0], (s3 & 7u) | 0x0c0c0c00u);
+  }
+  for (int d = 1; d < per; d <<= 1) bits += __shfl_xor(bits, d, per);
+  if (last)
+    atomicAdd(&s_words[off / (int64_t(chunk) * XP_LANES) - g_base],
+              static_cast<int32_t>((bits + XP_LIMIT - 1) / 32 + 1));
+}
+
+// The LUT from the lengths and codes, by a whole workgroup: a sixteenth of the
+// threads per symbol, which owns the windows whose low bits are its code.
+__device__ __forceinline__ void write_lut(const int32_t* s_len, const int32_t* s_code, uint8_t* lut, int threads) {
+  const int per = threads / code::kSyms, sym = threadIdx.x / per;
+  const int n = s_len[sym], code = s_code[sym];
+  for (int i = threadIdx.x % per; i < XP_LUT_BYTES >> n; i += per)
+    lut[code | (i << n)] = static_cast<uint8_t>((sym << 4) | n);
+}
+
+// ---- the plan of a row by several workgroups ----
+//
+// With a workspace the plan's two passes are launches of their own over
+// parts of the rows, so that a few rows fill the GPU and many rows leave no
+// partly empty round of one workgroup per row. One 2 MiB row: 266 us in one
+// workgroup, 7 + 12 us here; 256 rows: 316 us, 111 + 142 us (537 MB read
+// twice, at 4.8 and 3.8 TB/s; half of what was saved is the code's).
+
+// Exponent counts of part `blockIdx.x % parts` (kPartBytes values) of a row.
+// Each thread counts into its own LDS counters with atomic adds whose result
+// is not returned (see encode_plan_kernel).
+constexpr int64_t kPartBytes = 1 << 16;
+
+__global__ void __launch_bounds__(kThreads) encode_hist_kernel(EncodeArgs a) {
+  __shared__ uint32_t s_hist[code::kSyms][kThreads];
+  const int row = blockIdx.x / a.parts, part = blockIdx.x % a.parts;
+  const int tid = threadIdx.x;
+  const uint8_t* raw = a.raw + static_cast<int64_t>(row) * a.raw_stride;
+  const int64_t lo = part * kPartBytes, hi = lo + kPartBytes < a.n ? lo + kPartBytes : a.n;
+  constexpr int64_t kStep = int64_t(kThreads) * 16;
+  u32x4 v[kPlanUnroll];
+#pragma unroll
+  for (int u = 0; u < kPlanUnroll; ++u)
+    if (lo + tid * 16 + u * kStep < hi) v[u] = *reinterpret_cast<const u32x4*>(raw + lo + tid * 16 + u * kStep);
+  for (int s = 0; s < code::kSyms; ++s) s_hist[s][tid] = 0;
+  for (int64_t off0 = lo + tid * 16; off0 < hi; off0 += kStep * kPlanUnroll) {
+#pragma unroll
+    for (int u = 0; u < kPlanUnroll; ++u) {
+      if (off0 + u * kStep >= hi) continue;
+      const u32x4 x = v[u];
+      const int64_t next = off0 + (u + kPlanUnroll) * kStep;
+      if (next < hi) v[u] = *reinterpret_cast<const u32x4*>(raw + next);
+      const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) atomicAdd(&s_hist[(w[k] >> (8 * b + 3)) & 15u][tid], 1u);
+    }
+  }
+  __syncthreads();
+  // 16 threads per symbol, 16 counters each.
+  const int sym = tid >> 4, at = tid & 15;
+  uint32_t t = 0;
+#pragma unroll
+  for (int i = 0; i < kThreads / 16; ++i) t += s_hist[sym][at + 16 * i];
+#pragma unroll
+  for (int d = 8; d >= 1; d >>= 1) t += __shfl_xor(t, d, 16);
+  if (at == 0) a.hist[static_cast<int64_t>(blockIdx.x) * code::kSyms + sym] = t;
+}
+
+// The row's code from its parts' counts (each workgroup for itself; the
+// row's first one writes the LUT), then the Huffman words of `groups` groups
+// (1 to 8: as few as leave the launch within kWordsBlocks workgroups, so that
+// a row's code is not built many more times than there are groups in flight).
+constexpr int64_t kWordsBlocks = 2048;
+
+__global__ void __launch_bounds__(kThreads) encode_words_kernel(EncodeArgs a, int groups, int blocks_per_row) {
+  __shared__ int32_t s_len[code::kSyms];
+  __shared__ int32_t s_code[code::kSyms];
+  __shared__ int32_t s_words[kGroupsPerBlock];
+  const int row = blockIdx.x / blocks_per_row, part = blockIdx.x % blocks_per_row;
+  const int tid = threadIdx.x;
+  const uint8_t* raw = a.raw + static_cast<int64_t>(row) * a.raw_stride;
+  const int64_t group = int64_t(a.chunk) * XP_LANES;
+  const int64_t g0 = int64_t(part) * groups;
+  const int64_t lo = g0 * group, end = lo + groups * group, hi = end < a.n ? end : a.n;
+  constexpr int64_t kStep = int64_t(kThreads) * 16;
+  u32x4 v[kPlanUnroll];
+#pragma unroll
+  for (int u = 0; u < kPlanUnroll; ++u)
+    if (lo + tid * 16 + u * kStep < hi) v[u] = *reinterpret_cast<const u32x4*>(raw + lo + tid * 16 + u * kStep);
+  if (tid < 64) {
+    const uint32_t* h = a.hist + static_cast<int64_t>(row) * a.parts * code::kSyms + (tid & 15);
+    uint32_t t = 0;
+#pragma unroll 4
+    for (int i = tid >> 4; i < a.parts; i += 4) t += h[i * code::kSyms];
+    t += __shfl_xor(t, 16, 64);
+    t += __shfl_xor(t, 32, 64);
+    const int length = wave_code_lengths(t);
+    const int code = wave_canonical_code(length);
+    if (tid < code::kSyms) {
+      s_len[tid] = length;
+      s_code[tid] = code;
+    }
+  } else if (tid < 64 + kGroupsPerBlock) {
+    s_words[tid - 64] = 0;
+  }
+  __syncthreads();
+  if (part == 0) write_lut(s_len, s_code, a.lut + static_cast<int64_t>(row) * a.lut_stride, kThreads);
+  uint32_t lb[4];
+  pack_lengths(s_len, lb);
+  const int per = a.chunk / 16;
+  for (int64_t off0 = lo + tid * 16; off0 < hi; off0 += kStep * kPlanUnroll) {
+#pragma unroll
+    for (int u = 0; u < kPlanUnroll; ++u) {
+      const int64_t off = off0 + u * kStep;
+      if (off >= hi) continue;
+      const u32x4 x = v[u];
+      const int64_t next = off + kPlanUnroll * kStep;
+      if (next < hi) v[u] = *reinterpret_cast<const u32x4*>(raw + next);
+      add_chunk_words(x, off, a.chunk, per, lb, s_words, g0);
+    }
+  }
+  __syncthreads();
+  if (tid < groups && g0 + tid < a.G) a.words[static_cast<int64_t>(row) * a.G + g0 + tid] = s_words[tid];
+}
+
+// ---- the plan of a row by one workgroup ----
 __global__ void __launch_bounds__(kPlanThreads) encode_plan_kernel(EncodeArgs a) {
   __shared__ uint32_t s_hist[code::kSyms][kPlanThreads];  // per-thread counters
   __shared__ int32_t s_len[code::kSyms];
@@ -113,35 +353,20 @@ __global__ void __launch_bounds__(kPlanThreads) encode_plan_kernel(EncodeArgs a)
     if (part == 0) s_hist[sym][0] = t;
   }
   __syncthreads();
-  if (tid == 0) {
-    int64_t hist[code::kSyms];
-    for (int s = 0; s < code::kSyms; ++s) hist[s] = s_hist[s][0];
-    int32_t lengths[code::kSyms], codes[code::kSyms];
-    code::code_lengths(hist, lengths);
-    code::canonical_codes(lengths, codes);
-    for (int s = 0; s < code::kSyms; ++s) {
-      s_len[s] = lengths[s];
-      s_code[s] = codes[s];
+  if (tid < 64) {
+    const int length = wave_code_lengths(s_hist[tid & 15][0]);
+    const int code = wave_canonical_code(length);
+    if (tid < code::kSyms) {
+      s_len[tid] = length;
+      s_code[tid] = code;
     }
   }
   __syncthreads();
-  {
-    int32_t lengths[code::kSyms], codes[code::kSyms];
-    for (int s = 0; s < code::kSyms; ++s) {
-      lengths[s] = s_len[s];
-      codes[s] = s_code[s];
-    }
-    uint8_t* lut = a.lut + static_cast<int64_t>(row) * a.lut_stride;
-    for (int x = tid; x < XP_LUT_BYTES; x += kPlanThreads)
-      lut[x] = static_cast<uint8_t>(code::lut_entry(lengths, codes, x));
-  }
-  uint32_t lb[4] = {0u, 0u, 0u, 0u};  // the lengths as bytes, symbol s in byte s % 4 of lb[s / 4]
-#pragma unroll
-  for (int s = 0; s < code::kSyms; ++s) lb[s / 4] |= static_cast<uint32_t>(s_len[s]) << (8 * (s % 4));
+  write_lut(s_len, s_code, a.lut + static_cast<int64_t>(row) * a.lut_stride, kPlanThreads);
+  uint32_t lb[4];
+  pack_lengths(s_len, lb);
 
-  // 3. Words per chunk: (start bit of its last symbol + LIMIT - 1) / 32 + 1.
-  // The chunk's 16-byte pieces are spread over consecutive threads, so each
-  // chunk is summed by a power-of-two set of lanes of one wave.
+  // 3. Words per group.
   const int per = chunk / 16;  // threads per chunk
   for (int g = tid; g < G; g += kPlanThreads) s_words[g] = 0;
   __syncthreads();
@@ -156,17 +381,7 @@ __global__ void __launch_bounds__(kPlanThreads) encode_plan_kernel(EncodeArgs a)
     for (int u = 0; u < kPlanUnroll; ++u) {
       const int64_t off = off0 + u * kStep;
       if (off >= n) continue;
-      uint32_t bits = sum_lengths4(v[u].x, lb) + sum_lengths4(v[u].y, lb) + sum_lengths4(v[u].z, lb) +
-                      sum_lengths4(v[u].w, lb);
-      const bool last = ((off + 16) % chunk) == 0;
-      if (last) {  // not the last symbol
-        const uint32_t s3 = v[u].w >> 27 & 15u;
-        const bool hi = s3 >= 8u;
-        bits -= __builtin_amdgcn_perm(hi ? lb[3] : lb[1], hi ? lb[2] : lb[0], (s3 & 7u) | 0x0c0c0c00u);
-      }
-      for (int d = 1; d < per; d <<= 1) bits += __shfl_xor(bits, d, per);
-      if (last)
-        atomicAdd(&s_words[off / (int64_t(chunk) * XP_LANES)], static_cast<int32_t>((bits + XP_LIMIT - 1) / 32 + 1));
+      add_chunk_words(v[u], off, chunk, per, lb, s_words, 0);
     }
   }
   __syncthreads();
@@ -192,18 +407,69 @@ __global__ void __launch_bounds__(kPlanThreads) encode_plan_kernel(EncodeArgs a)
   for (int64_t i = nbytes / 4 + tid; i < a.pitch / 4; i += kPlanThreads) reinterpret_cast<uint32_t*>(rec)[i] = 0;
 }
 
+// SPLIT: the words per group come from encode_words_kernel; the workgroup
+// sums those before its groups and writes its part of gstart and of the tail.
+template <bool SPLIT>
 __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, int blocks_per_row) {
   __shared__ int32_t s_len[code::kSyms];
   __shared__ uint32_t s_tab[code::kSyms];  // code | length << 16
+  __shared__ int32_t s_gstart[kGroupsPerBlock + 1];  // SPLIT: of the workgroup's groups, then the row's words
+  __shared__ int32_t s_sum[2][kThreads / 64];
 
   const int row = blockIdx.x / blocks_per_row, part = blockIdx.x % blocks_per_row;
   const int tid = threadIdx.x;
-  if (a.needed[row] > a.pitch) return;  // the row does not fit: the plan wrote nothing either
   const uint8_t* raw = a.raw + static_cast<int64_t>(row) * a.raw_stride;
   uint8_t* rec = a.rec + static_cast<int64_t>(row) * a.pitch;
   const int64_t n = a.n;
   const int chunk = a.chunk, G = a.G;
-  const int32_t* gstart = reinterpret_cast<const int32_t*>(rec);
+  const int gfirst = part * kGroupsPerBlock;
+  const int64_t head = 4 * (int64_t(G) + 1) + n / 2;
+  if constexpr (SPLIT) {
+    const int32_t* words = a.words + static_cast<int64_t>(row) * G;
+    int32_t below = 0, all = 0;
+    for (int g = tid; g < G; g += kThreads) {
+      const int32_t w = words[g];
+      all += w;
+      below += g < gfirst ? w : 0;
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+      all += __shfl_xor(all, d, 64);
+      below += __shfl_xor(below, d, 64);
+    }
+    if ((tid & 63) == 0) {
+      s_sum[0][tid >> 6] = below;
+      s_sum[1][tid >> 6] = all;
+    }
+    __syncthreads();
+    below = all = 0;
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) {
+      below += s_sum[0][w];
+      all += s_sum[1][w];
+    }
+    const int64_t nbytes = head + 4 * int64_t(all);
+    if (tid == 0 && part == 0) a.needed[row] = nbytes;
+    if (nbytes > a.pitch) return;  // the row does not fit: only its LUT and its size are written
+    if (tid < kGroupsPerBlock) {
+      for (int i = 0; i < tid; ++i) below += gfirst + i < G ? words[gfirst + i] : 0;
+      s_gstart[tid] = below;
+      if (gfirst + tid < G) reinterpret_cast<int32_t*>(rec)[gfirst + tid] = below;
+    } else if (tid == kGroupsPerBlock) {
+      s_gstart[tid] = all;
+      if (part == 0) reinterpret_cast<int32_t*>(rec)[G] = all;
+    }
+    // Zero tail (nbytes and the pitch are multiples of 4), a stride per workgroup.
+    for (int64_t i = nbytes / 4 + int64_t(part) * kThreads + tid; i < a.pitch / 4; i += int64_t(blocks_per_row) * kThreads)
+      reinterpret_cast<uint32_t*>(rec)[i] = 0;
+  } else {
+    if (a.needed[row] > a.pitch) return;  // the row does not fit: the plan wrote nothing either
+    const int32_t* gstart = reinterpret_cast<const int32_t*>(rec);
+    if (tid < kGroupsPerBlock)
+      s_gstart[tid] = gstart[gfirst + tid < G ? gfirst + tid : G];
+    else if (tid == kGroupsPerBlock)
+      s_gstart[tid] = gstart[G];
+  }
 
   // 4. The code from the LUT (entry = symbol << 4 | length), then groups,
   // one per half-wave.
@@ -213,16 +479,13 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
     s_len[ent >> 4] = static_cast<int32_t>(ent & 15u);  // every entry of a symbol holds the same length
   }
   __syncthreads();
-  if (tid == 0) {
-    int32_t lengths[code::kSyms], codes[code::kSyms];
-    for (int s = 0; s < code::kSyms; ++s) lengths[s] = s_len[s];
-    code::canonical_codes(lengths, codes);
-    for (int s = 0; s < code::kSyms; ++s)
-      s_tab[s] = static_cast<uint32_t>(codes[s]) | (static_cast<uint32_t>(lengths[s]) << 16);
+  if (tid < 64) {
+    const int length = s_len[tid & 15];
+    const int code = wave_canonical_code(length);
+    if (tid < code::kSyms) s_tab[tid] = static_cast<uint32_t>(code) | (static_cast<uint32_t>(length) << 16);
   }
   __syncthreads();
 
-  const int64_t head = 4 * (int64_t(G) + 1) + n / 2;
   uint32_t* fixed = reinterpret_cast<uint32_t*>(rec + 4 * (int64_t(G) + 1));
   uint32_t* huff = reinterpret_cast<uint32_t*>(rec + head);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -230,9 +493,9 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
   const uint32_t li = lane & 31;
   const uint32_t half_shift = upper ? 16u : 0u;
   const int mwords = chunk / 8;
-  const uint32_t total = static_cast<uint32_t>(gstart[G]);  // every word position is below it
+  const uint32_t total = static_cast<uint32_t>(s_gstart[kGroupsPerBlock]);  // every word position is below it
   {
-    const int g0 = part * kGroupsPerBlock + 2 * wave;
+    const int g0 = gfirst + 2 * wave;
     if (g0 >= G) return;
     const int g = g0 + (upper ? 1 : 0);
     const bool live = g < G;  // a spare half-wave walks the last group and writes nothing
@@ -246,8 +509,8 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
     // half's refills of a symbol (at most 32) never borrows. A lane's
     // queued positions are relative; gbase makes them absolute.
     constexpr uint32_t kBias = 64;
-    const uint32_t gs_lo = static_cast<uint32_t>(gstart[g0]);
-    const uint32_t gs_hi = static_cast<uint32_t>(gstart[g0 + 1 < G ? g0 + 1 : G - 1]);
+    const uint32_t gs_lo = static_cast<uint32_t>(s_gstart[2 * wave]);
+    const uint32_t gs_hi = static_cast<uint32_t>(s_gstart[2 * wave + (g0 + 1 < G ? 1 : 0)]);
     const uint32_t gbase = upper ? gs_hi - kBias : gs_lo;
     uint32_t offs = kBias << 16;
     uint32_t level = 0;         // bits the decoder has buffered
@@ -336,6 +599,8 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
   }
 }
 
+int64_t hist_parts(int64_t n) { return (n + kPartBytes - 1) / kPartBytes; }
+
 }  // namespace
 }  // namespace xp
 
@@ -343,8 +608,20 @@ using namespace xp;
 
 extern "C" {
 
+int64_t xp_encode_workspace_bytes(int64_t rows, int64_t n, int64_t chunk) {
+  if (rows <= 0 || n <= 0 || chunk <= 0) return 0;
+  return 4 * rows * (hist_parts(n) * code::kSyms + n / (chunk * XP_LANES));
+}
+
 int xp_encode_rows(const uint8_t* raw, int64_t rows, int64_t raw_stride, int64_t n, int64_t chunk, uint8_t* records,
                    int64_t pitch, uint8_t* luts, int64_t lut_stride, int64_t* needed, void* stream) {
+  return xp_encode_rows_split(raw, rows, raw_stride, n, chunk, records, pitch, luts, lut_stride, needed, nullptr, 0,
+                              stream);
+}
+
+int xp_encode_rows_split(const uint8_t* raw, int64_t rows, int64_t raw_stride, int64_t n, int64_t chunk,
+                         uint8_t* records, int64_t pitch, uint8_t* luts, int64_t lut_stride, int64_t* needed,
+                         void* work, int64_t work_bytes, void* stream) {
   XP_REQUIRE(rows >= 0 && rows <= INT32_MAX, "xp_encode_rows: rows=%lld", (long long)rows);
   if (rows == 0) return XP_OK;
   XP_REQUIRE(raw && records && luts && needed, "xp_encode_rows: null argument");
@@ -363,14 +640,41 @@ int xp_encode_rows(const uint8_t* raw, int64_t rows, int64_t raw_stride, int64_t
              "xp_encode_rows: pitch %lld is not a positive multiple of 16", (long long)pitch);
   XP_REQUIRE(lut_stride >= XP_LUT_BYTES, "xp_encode_rows: lut_stride=%lld", (long long)lut_stride);
   EncodeArgs a{raw, raw_stride, n, static_cast<int>(chunk), static_cast<int>(G), records, pitch,
-               luts, lut_stride, needed};
+               luts, lut_stride, needed, nullptr, nullptr, 0};
   const int64_t blocks = (G + kGroupsPerBlock - 1) / kGroupsPerBlock;
   XP_REQUIRE(rows * blocks <= INT32_MAX, "xp_encode_rows: %lld rows x %lld blocks", (long long)rows, (long long)blocks);
-  hipLaunchKernelGGL(encode_plan_kernel, dim3(static_cast<unsigned>(rows)), dim3(kPlanThreads), 0, as_stream(stream),
-                     a);
-  if (int rc = check_launch("encode_plan_kernel")) return rc;
-  hipLaunchKernelGGL(encode_groups_kernel, dim3(static_cast<unsigned>(rows * blocks)), dim3(kThreads), 0,
-                     as_stream(stream), a, static_cast<int>(blocks));
+  const dim3 grid(static_cast<unsigned>(rows * blocks));
+  if (!work) {
+    hipLaunchKernelGGL(encode_plan_kernel, dim3(static_cast<unsigned>(rows)), dim3(kPlanThreads), 0,
+                       as_stream(stream), a);
+    if (int rc = check_launch("encode_plan_kernel")) return rc;
+    hipLaunchKernelGGL(encode_groups_kernel<false>, grid, dim3(kThreads), 0, as_stream(stream), a,
+                       static_cast<int>(blocks));
+    return check_launch("encode_groups_kernel");
+  }
+  const int64_t need = xp_encode_workspace_bytes(rows, n, chunk);
+  XP_REQUIRE(work_bytes >= need && (reinterpret_cast<uintptr_t>(work) & 3) == 0,
+             "xp_encode_rows_split: workspace of %lld B, needs %lld, 4-byte aligned", (long long)work_bytes,
+             (long long)need);
+  const int64_t parts = hist_parts(n);
+  XP_REQUIRE(rows * parts <= INT32_MAX, "xp_encode_rows_split: %lld rows x %lld parts", (long long)rows,
+             (long long)parts);
+  a.parts = static_cast<int>(parts);
+  a.hist = static_cast<uint32_t*>(work);
+  a.words = static_cast<int32_t*>(work) + rows * parts * code::kSyms;
+  hipLaunchKernelGGL(encode_hist_kernel, dim3(static_cast<unsigned>(rows * parts)), dim3(kThreads), 0,
+                     as_stream(stream), a);
+  if (int rc = check_launch("encode_hist_kernel")) return rc;
+  int64_t groups = 1;
+  while (groups < kGroupsPerBlock && rows * ((G + groups - 1) / groups) > kWordsBlocks) groups *= 2;
+  const int64_t word_blocks = (G + groups - 1) / groups;
+  XP_REQUIRE(rows * word_blocks <= INT32_MAX, "xp_encode_rows_split: %lld rows x %lld blocks", (long long)rows,
+             (long long)word_blocks);
+  hipLaunchKernelGGL(encode_words_kernel, dim3(static_cast<unsigned>(rows * word_blocks)), dim3(kThreads), 0,
+                     as_stream(stream), a, static_cast<int>(groups), static_cast<int>(word_blocks));
+  if (int rc = check_launch("encode_words_kernel")) return rc;
+  hipLaunchKernelGGL(encode_groups_kernel<true>, grid, dim3(kThreads), 0, as_stream(stream), a,
+                     static_cast<int>(blocks));
   return check_launch("encode_groups_kernel");
 }
 

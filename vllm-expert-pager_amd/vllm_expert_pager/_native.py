@@ -137,6 +137,8 @@ _SIGNATURES = {
     "xp_moe_layer_bytes": (_L, [_L, _L, _L, _L, _L]),
     "xp_moe_layer": (_I, [_P, _L, _L, _P, _I, _L, _P, _P, _L, _L, _P, _P, _P, _P, _L, _P, _L, _P, _I, _P]),
     "xp_encode_rows": (_I, [_P, _L, _L, _L, _L, _P, _L, _P, _L, _P, _P]),
+    "xp_encode_workspace_bytes": (_L, [_L, _L, _L]),
+    "xp_encode_rows_split": (_I, [_P, _L, _L, _L, _L, _P, _L, _P, _L, _P, _P, _L, _P]),
     "xp_moe_topk_sum": (_I, [_P, _L, _L, _L, _P, _I, _L, _P, _P]),
 }
 

@@ -75,7 +75,7 @@ def encode_into(raw: np.ndarray, record: np.ndarray, lut: np.ndarray, chunk: int
 
 def encode_rows(raw: torch.Tensor, pitch: int, chunk: int = CHUNK, records: torch.Tensor | None = None,
                 luts: torch.Tensor | None = None, check: bool = True) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """Compress the uint8 rows ``raw`` (R, N) on the GPU, one workgroup per row (codec.py:125-193).
+    """Compress the uint8 rows ``raw`` (R, N) on the GPU (codec.py:125-193).
 
     Returns ``(records (R, pitch), luts (R, 512), needed (R,) int64)`` on raw's
     device, byte for byte what ``encode_into`` writes. With ``check`` (it
@@ -98,8 +98,10 @@ def encode_rows(raw: torch.Tensor, pitch: int, chunk: int = CHUNK, records: torc
     if records.stride(0) != pitch:
         raise ValueError("records rows must be contiguous at the pitch")
     needed = torch.empty((R,), dtype=torch.int64, device=raw.device)
-    nat.call("xp_encode_rows", raw.data_ptr(), R, raw.stride(0), N, chunk, records.data_ptr(), pitch,
-             luts.data_ptr(), luts.stride(0), needed.data_ptr(), nat.stream())
+    nbytes = int(nat.lib().xp_encode_workspace_bytes(R, N, chunk))
+    work = torch.empty((max(nbytes, 4),), dtype=torch.uint8, device=raw.device)
+    nat.call("xp_encode_rows_split", raw.data_ptr(), R, raw.stride(0), N, chunk, records.data_ptr(), pitch,
+             luts.data_ptr(), luts.stride(0), needed.data_ptr(), work.data_ptr(), nbytes, nat.stream())
     if check and R:
         worst = int(needed.max().item())
         if worst > pitch:

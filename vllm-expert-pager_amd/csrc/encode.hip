@@ -15,11 +15,11 @@
 //      most LIMIT bits, so each one appears in the 9-bit table with its
 //      length, and the canonical codes follow from the lengths); then each
 //      32-lane half-wave encodes one group: its lanes walk their chunks
-//      in lockstep, run the decoder's refill rule, and give each word the
-//      (symbol index, lane) rank of its refill -- the wave ballot's count of
-//      refilling lanes below, as the decoder computes it. A lane emits a
-//      word once its 32 bits are complete; at most two refills are waiting
-//      for their word. The lane also writes its sign/mantissa nibble words.
+//      in lockstep, two symbols at a time, run the decoder's refill rule, and
+//      give each word the (symbol index, lane) rank of its refill -- the wave
+//      ballot's count of refilling lanes below, as the decoder computes it. A
+//      lane emits a word once its 32 bits are complete. The lane also writes
+//      its sign/mantissa nibble words.
 // The record is written whole: nibbles and Huffman words by the groups
 // launch, gstart and the zero tail up to the pitch by it or by
 // encode_plan_kernel. A row that does not fit its pitch writes nothing but its
@@ -412,7 +412,8 @@ __global__ void __launch_bounds__(kPlanThreads) encode_plan_kernel(EncodeArgs a)
 template <bool SPLIT>
 __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, int blocks_per_row) {
   __shared__ int32_t s_len[code::kSyms];
-  __shared__ uint32_t s_tab[code::kSyms];  // code | length << 16
+  __shared__ uint32_t s_code[code::kSyms];  // code | length << 16
+  __shared__ uint2 s_pair[code::kSyms * code::kSyms];  // see encode_pair
   __shared__ int32_t s_gstart[kGroupsPerBlock + 1];  // SPLIT: of the workgroup's groups, then the row's words
   __shared__ int32_t s_sum[2][kThreads / 64];
 
@@ -482,7 +483,14 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
   if (tid < 64) {
     const int length = s_len[tid & 15];
     const int code = wave_canonical_code(length);
-    if (tid < code::kSyms) s_tab[tid] = static_cast<uint32_t>(code) | (static_cast<uint32_t>(length) << 16);
+    if (tid < code::kSyms) s_code[tid] = static_cast<uint32_t>(code) | (static_cast<uint32_t>(length) << 16);
+  }
+  __syncthreads();
+  static_assert(kThreads == code::kSyms * code::kSyms, "a thread per pair of symbols");
+  {
+    const uint32_t first = s_code[tid & 15], second = s_code[tid >> 4];
+    const uint32_t l0 = first >> 16, l01 = l0 + (second >> 16);
+    s_pair[tid] = make_uint2((first & 0xffffu) | ((second & 0xffffu) << l0), (l0 << 26) | l01);
   }
   __syncthreads();
 
@@ -506,18 +514,70 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
     // words are at most 32 chunks of 9-bit codes), packed in one scalar
     // register: the lower half's in bits 0-15, the upper half's in 16-31
     // biased by kBias, so that lowering the upper half's count by the lower
-    // half's refills of a symbol (at most 32) never borrows. A lane's
-    // queued positions are relative; gbase makes them absolute.
+    // half's refills of a symbol (at most 32) never borrows. A lane's word
+    // positions are relative; gbase makes them absolute.
     constexpr uint32_t kBias = 64;
     const uint32_t gs_lo = static_cast<uint32_t>(s_gstart[2 * wave]);
     const uint32_t gs_hi = static_cast<uint32_t>(s_gstart[2 * wave + (g0 + 1 < G ? 1 : 0)]);
     const uint32_t gbase = upper ? gs_hi - kBias : gs_lo;
+    const uint32_t limit = live ? total : 0u;
     uint32_t offs = kBias << 16;
-    uint32_t level = 0;         // bits the decoder has buffered
-    uint64_t acc = 0;           // bits of the lane's stream not yet emitted
-    uint32_t accbits = 0;
-    uint32_t q0 = 0, q1 = 0;    // positions of words refilled but not yet emitted
-    uint32_t qn = 0;
+    // The decoder has fewer than LIMIT bits left before the symbol that starts
+    // at bit P of the lane's stream exactly when the words it has loaded
+    // number no more than (P + LIMIT - 1) / 32, so it loads one where that
+    // quotient steps: where bit 5 of Q = P + LIMIT - 1 differs from the
+    // symbol's before it (a symbol is shorter than 32 bits). Q mod 64 is kept
+    // in bits 26-31, so that the step is a sign. The first symbol always
+    // loads.
+    uint32_t Q = uint32_t(XP_LIMIT - 1) << 26;  // of the next symbol
+    uint32_t Qp = Q ^ 0x80000000u;              // of the symbol before (bits below 26 are not used)
+    uint32_t acc = 0, accbits = 0;              // the bits of the word being filled
+    uint32_t wcur = 0, wprev = 0;               // positions of the last word loaded and the one before
+    // Two symbols at a time (`at` is 8 x (second * 16 + first)): a pair's
+    // entry holds both codes in a row, their length l01 in bits 0-5 and the
+    // first's in bits 26-31. Loads are at least three symbols apart (a load
+    // leaves 32 bits or more, a symbol takes at most 9), so a pair has at
+    // most one; and at most 18 bits, so it completes at most one word. That
+    // word is the last one loaded, unless the next one has been loaded
+    // already, as soon as 24 of its bits are there: unless the second symbol
+    // starts before bit 24. Completing a word from a start of at most 23 takes
+    // all 9 bits from exactly 23, where Q mod 32 = 31.
+    // The loop is VALU bound: about 20 instructions a symbol, half of what
+    // symbol by symbol with a two-entry queue of loaded words took. 256 rows
+    // of 2 MiB: 485 -> 358 us (2.2 TB/s read and written); one row, a chain of
+    // 512 symbols in 64 waves, 71 -> 48 us. Reading a 16-byte piece's eight
+    // entries ahead of its pairs changed neither.
+    auto encode_pair = [&](uint32_t at) {
+      const uint2 t = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(s_pair) + at);
+      const uint32_t q1 = Q + t.y;
+      const bool r0 = static_cast<int32_t>(Q ^ Qp) < 0, r1 = static_cast<int32_t>(q1 ^ Q) < 0;
+      auto place = [&](bool refill) {  // the word's rank among the refilling lanes of the half
+        const unsigned long long mask = __builtin_amdgcn_ballot_w64(refill);
+        const uint32_t m_lo = static_cast<uint32_t>(mask), m_hi = static_cast<uint32_t>(mask >> 32);
+        const uint32_t n_lo = static_cast<uint32_t>(__popc(m_lo)), n_hi = static_cast<uint32_t>(__popc(m_hi));
+        const uint32_t bases = offs - (n_lo << 16);
+        offs += n_lo + (n_hi << 16);
+        return __builtin_amdgcn_mbcnt_hi(
+            m_hi, __builtin_amdgcn_mbcnt_lo(m_lo, __builtin_amdgcn_ubfe(bases, half_shift, 16u)));
+      };
+      const uint32_t p0 = place(r0), p1 = place(r1);
+      wprev = r0 || r1 ? wcur : wprev;
+      wcur = r0 ? p0 : wcur;
+      wcur = r1 ? p1 : wcur;
+      Q += t.y << 26;
+      Qp = q1;
+      const uint64_t shifted = static_cast<uint64_t>(t.x) << accbits;
+      const uint32_t word = acc | static_cast<uint32_t>(shifted);
+      const uint32_t bits = accbits + (t.y & 63u);
+      const bool full = bits >= 32;
+      if (full) {
+        const bool alone = (q1 & 0x7C000000u) == 0x7C000000u;
+        const uint32_t at_word = gbase + (alone ? wcur : wprev);
+        if (at_word < limit) huff[at_word] = word;
+      }
+      acc = full ? static_cast<uint32_t>(shifted >> 32) : word;
+      accbits = bits & 31u;
+    };
     // A lane's values in blocks of 64 (four 16-byte loads back to back, so
     // each cache line of its chunk is fetched about twice instead of once
     // per 16 values), the next block loaded while this one is encoded.
@@ -526,7 +586,6 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (j < nv) cur[j] = *reinterpret_cast<const u32x4*>(src + 16 * j);
-    const uint8_t* tab = reinterpret_cast<const uint8_t*>(s_tab);
     for (int i0 = 0; i0 < chunk; i0 += 16 * nv) {
       if (i0 + 16 * nv < chunk) {
 #pragma unroll
@@ -541,37 +600,11 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          // Each byte's exponent field (bits 3-6) as a byte offset into s_tab.
-          const uint32_t ex4 = (w[k] >> 1) & 0x3C3C3C3Cu;
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            // The decoder's refill rule: a lane with fewer than LIMIT bits
-            // buffered takes the next word of its group, ranked by the
-            // refilling lanes below it in its half.
-            const bool refill = level < static_cast<uint32_t>(XP_LIMIT);
-            const unsigned long long mask = __builtin_amdgcn_ballot_w64(refill);
-            const uint32_t m_lo = static_cast<uint32_t>(mask), m_hi = static_cast<uint32_t>(mask >> 32);
-            const uint32_t n_lo = static_cast<uint32_t>(__popc(m_lo)), n_hi = static_cast<uint32_t>(__popc(m_hi));
-            const uint32_t bases = offs - (n_lo << 16);
-            const uint32_t pos = __builtin_amdgcn_mbcnt_hi(
-                m_hi, __builtin_amdgcn_mbcnt_lo(m_lo, __builtin_amdgcn_ubfe(bases, half_shift, 16u)));
-            offs += n_lo + (n_hi << 16);
-            q0 = refill && qn == 0 ? pos : q0;
-            q1 = refill && qn != 0 ? pos : q1;
-            qn += refill ? 1u : 0u;
-            level += refill ? 32u : 0u;
-            const uint32_t t = *reinterpret_cast<const uint32_t*>(tab + __builtin_amdgcn_ubfe(ex4, 8u * b, 8u));
-            const uint32_t len = t >> 16;
-            acc |= static_cast<uint64_t>(t & 0xffffu) << accbits;
-            accbits += len;
-            level -= len;
-            const bool full = accbits >= 32;  // word q0 is complete
-            if (full && live && gbase + q0 < total) huff[gbase + q0] = static_cast<uint32_t>(acc);
-            acc = full ? acc >> 32 : acc;
-            accbits &= 31u;  // below 32 + LIMIT
-            q0 = full ? q1 : q0;
-            qn -= full ? 1u : 0u;
-          }
+          // A byte's exponent field is bits 3-6: the pairs' table offsets are
+          // bits 3-10 and 19-26 of the fields and the fields shifted down by 4.
+          const uint32_t ex = w[k] & 0x78787878u, z = ex | (ex >> 4);
+          encode_pair(z & 0x7F8u);
+          encode_pair((z >> 16) & 0x7F8u);
           if (k & 1) {  // 8 values: one nibble word, value j in bits 4j..4j+3
             // Per byte, sign (bit 7) to bit 3 beside the mantissa (bits 0-2);
             // then two bytes' nibbles joined and the four pairs picked.
@@ -586,15 +619,15 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
 #pragma unroll
       for (int j = 0; j < 4; ++j) cur[j] = nxt[j];
     }
-    // Words whose refill came but whose bits ran out: the rest of the stream,
-    // then zeros.
-    while (__builtin_amdgcn_ballot_w64(qn > 0)) {
-      if (qn > 0) {
-        if (live && gbase + q0 < total) huff[gbase + q0] = static_cast<uint32_t>(acc);
-        acc >>= 32;
-        q0 = q1;
-        --qn;
-      }
+    // Words loaded and not complete: the one being filled if the last symbol
+    // started at or after bit 1 - LIMIT = -8 of it, and the next one, all
+    // zeros, if it started at or after bit 24.
+    const int last = static_cast<int>(accbits) - static_cast<int>((Q - (Qp & 0xFC000000u)) >> 26);
+    if (last >= 24) {
+      if (gbase + wprev < limit) huff[gbase + wprev] = acc;
+      if (gbase + wcur < limit) huff[gbase + wcur] = 0;
+    } else if (last >= -8) {
+      if (gbase + wcur < limit) huff[gbase + wcur] = acc;
     }
   }
 }

@@ -497,3 +497,28 @@ def test_fused_moe_equals_separate_calls(T, topk, E, S, mapped, num, idbits):
     # The same ids as strided views and weights in another type.
     wide = torch.stack([ids_t, ids_t], dim=2)[:, :, 0]
     assert torch.equal(moe.fused_moe(xb, tw_t.double(), wide, *w, expert_map=emap, num_experts=num), out)
+
+
+# The gate/up launch takes 4, 8 or 16 rows of a slot by the token count: each
+# side of those lines, slots with more pairs than rows (every token on the
+# same experts, and one expert named by every pair), an odd number of columns
+# blocks, and a one-slot slab.
+@pytest.mark.parametrize("T, topk, E, route", [(1, 10, 12, "random"), (3, 8, 300, "random"), (4, 8, 8, "same"),
+                                               (5, 8, 8, "same"), (8, 8, 40, "random"), (8, 8, 40, "one"),
+                                               (9, 7, 9, "same"), (4, 16, 20, "one"), (21, 3, 5, "same"),
+                                               (64, 1, 1, "one")])
+def test_decode_rows_by_token_count(T, topk, E, route):
+    moe = _moe()
+    H, I = 640, 384
+    x, tw, _, w13, w13s, w2, w2s = _case(T + E, E, H, I, T, topk)
+    rng = np.random.default_rng(T)
+    ids = np.stack([rng.permutation(E)[:topk] if topk <= E else rng.integers(0, E, topk) for _ in range(T)])
+    if route == "same":
+        ids[:] = ids[0]
+    elif route == "one":
+        ids[:] = E - 1
+    xb, emap = _bf16(x), torch.arange(E, dtype=torch.int32, device="cuda").flip(0).contiguous()
+    tw_t, ids_t, *w = _dev(tw, ids, w13, w13s, w2, w2s)
+    want = _separate(moe, xb, tw_t, ids_t, emap, E, E, w)
+    got = moe.decode_experts(xb, tw_t, ids_t, emap, E, *w, E)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

@@ -1123,14 +1123,13 @@ __global__ void __launch_bounds__(kThreads) gemm1_narrow_kernel(const uint8_t* _
 // For at most kDecodePairs pairs, every wave of every gemm1 workgroup routes
 // the pairs itself (one pair per lane) and the workgroup quantises the token
 // rows it multiplies into LDS, so no routing or quantisation launch precedes
-// it. gemm2 then takes one token and 8 output columns per workgroup, computes
+// it. gemm2 then takes one token and 8 or 16 output columns per workgroup, computes
 // each of the token's pairs and sums them there, so no top-k sum launch
 // follows. The bits are those of xp_moe_quant_route, xp_moe_experts and
 // xp_moe_topk_sum.
 constexpr int kDecodePairs = 64;
 constexpr int kDecodeMaxH = 4096;       // 16 quantised token rows of H bytes fit in LDS
 constexpr int kDecodeActBytes = 32768;  // a token's quantised activations (topk x I) in LDS
-constexpr int kDecodeCols2 = 8;         // output columns per gemm2_decode_kernel workgroup
 
 // Pair p's slot (-1: an id outside [0, E) or an expert without a slot):
 // from the acquire's per-pair slots when given, else ids then expert_map.
@@ -1147,42 +1146,51 @@ __device__ __forceinline__ int decode_slot(int p, int n, const void* ids, int eb
   return p < n && sl >= 0 && sl < slots ? sl : -1;
 }
 
-// The step's routing as route_kernel lists it (pairs by slot, then by pair
-// index; one tile per occupied slot, since a slot holds at most 64 of these
-// pairs), computed by one wave from the pairs' slots (lane p: pair p): on
-// the lane of each slot's first pair, the slot's 16-row subtiles (nsub) and
-// the index of its first one among all the step's subtiles in slot order
-// (start); zero subtiles on the other lanes. The loops run over uniform pair
-// indices, so each read of another lane's value is a readlane.
+// The step's routing, computed by one wave from the pairs' slots (lane p:
+// pair p): on the lane of each slot's first pair, the slot's ROWS-row subtiles
+// (nsub) and the index of its first one among all the step's subtiles, in the
+// order of the slots' first pairs (start); zero subtiles on the other lanes.
+// The lanes of one slot are found bit by bit of the slot number, so the cost
+// is the bits of `slots`, not the pairs: every wave of every workgroup routes,
+// and readlane loops over 32 pairs took 3 us of a 4-token step's 21.
 struct DecodeRoute {
-  int slot, start, nsub;
+  int start, nsub;
 };
 
-__device__ __forceinline__ DecodeRoute decode_route(int slot, int n) {
-  const int lane = threadIdx.x & 63;
-  bool first = slot >= 0;
-  int count = 0;
-  for (int q = 0; q < n; ++q) {
-    const int sq = __builtin_amdgcn_readlane(slot, q);
-    if (q < lane && sq == slot) first = false;
-    count += sq == slot ? 1 : 0;
+template <int ROWS>
+__device__ __forceinline__ DecodeRoute decode_route(int slot, int slots) {
+  unsigned long long same = __ballot(slot >= 0);
+  const int bits = 32 - __clz(slots - 1);  // of slots 0 .. slots - 1
+  for (int b = 0; b < bits; ++b) {
+    const bool set = (slot >> b) & 1;
+    const unsigned long long m = __ballot(set);
+    same &= set ? m : ~m;
   }
-  const int nsub = first ? (count + 15) >> 4 : 0;
+  const int count = slot >= 0 ? __popcll(same) : 0;
+  const bool first = slot >= 0 && lane_prefix(same) == 0;
+  const int nsub = first ? (count + ROWS - 1) / ROWS : 0;
   int start = 0;
-  for (int q = 0; q < n; ++q) {
-    const int sq = __builtin_amdgcn_readlane(slot, q), nq = __builtin_amdgcn_readlane(nsub, q);
-    if (sq < slot) start += nq;
-  }
-  return DecodeRoute{slot, start, nsub};
+#pragma unroll
+  for (int b = 0; (kDecodePairs / ROWS) >> b; ++b)
+    start += static_cast<int>(lane_prefix(__ballot((nsub >> b) & 1))) << b;
+  return DecodeRoute{start, nsub};
 }
 
 // gemm1_narrow_kernel over a decode step's pairs, with their routing and the
-// quantisation of their token rows done here. Dynamic LDS: 16 x H fp8 rows.
+// quantisation of their token rows done here. Dynamic LDS: the fp8 token rows.
 // Every wave routes the step itself (a pair per lane), so the weight rows of
 // the workgroup's slot are requested as soon as the pairs' slots arrive; the
-// token rows, requested before the slots, are quantised while the weights
-// are in flight.
-template <int ACT>
+// token rows, requested before them (one or two tokens: before the slots),
+// are quantised while the weights are in flight.
+//
+// A workgroup takes ROWS pairs of a slot (the product always has 16 rows;
+// those past ROWS are not kept). A few tokens give a slot a few pairs at
+// most, and the LDS of 16 rows (32 KB of token rows at H = 2048, 32 KB of
+// products) let only two workgroups share a CU, so that a step of 4 tokens
+// ran in two rounds of load latencies. 4 tokens, 32 of 256 experts 2048 x
+// 512: 25 -> 21 us with 4 rows, 16 us with the shorter routing (67 MB of
+// weights: 2.7 -> 4.2 TB/s).
+template <int ACT, int ROWS>
 __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
     const uint16_t* __restrict__ x, int64_t H, int64_t I, const void* ids, int eb, int npairs, int topk,
     const int32_t* __restrict__ expert_map, const int32_t* __restrict__ pair_slot, int E, int slots,
@@ -1190,17 +1198,19 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
     const float* __restrict__ w13_scale, Work work) {
   constexpr int kPerWave = kSplitRound / (kThreads / 64);
   constexpr int kPre = 4;  // token pieces per thread requested before the routing
-  extern __shared__ __attribute__((aligned(16))) uint8_t s_aq[];  // [16][H] fp8 token rows
-  __shared__ int s_pair[16];
-  __shared__ int s_arow[16];            // LDS row of each subtile row's activations
-  __shared__ float s_xs[16 * kMaxKB];   // their scales [LDS row][K block]
+  constexpr int kLanes = 4 * ROWS;  // lanes 16q + j whose product rows 4q .. 4q + 3 are below ROWS
+  static_assert(ROWS == 4 || ROWS == 8 || ROWS == 16, "whole 4-row groups of the product");
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_aq[];  // [rows][H] fp8 token rows
+  __shared__ int s_pair[ROWS];
+  __shared__ int s_arow[16];             // LDS row of each product row's activations
+  __shared__ float s_xs[ROWS * kMaxKB];  // their scales [LDS row][K block]
   __shared__ float s_sw[2][kMaxKB];
-  __shared__ float s_m[16];
+  __shared__ float s_m[ROWS];
   // Raw products of a round: [K block][gate, up][row within the lane's
   // 4-row group][lane], so that a wave reads its own row's values in lane
   // order.
-  __shared__ float s_part[kSplitRound][2][4][64];
-  __shared__ __attribute__((aligned(16))) uint16_t s_o[16 * 16];
+  __shared__ float s_part[kSplitRound][2][4][kLanes];
+  __shared__ __attribute__((aligned(16))) uint16_t s_o[ROWS * 16];
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int q = lane >> 4, j = lane & 15;
@@ -1237,7 +1247,8 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
   // hundreds of workgroups: 143 against 31 us at 8 tokens).
   const int ntok = npairs / topk;
   const bool by_token = ntok <= 2;
-  const int nc8 = static_cast<int>(H / 8), npiece = by_token ? ntok * nc8 : 0;
+  const int nc8 = static_cast<int>(H / 8);
+  int npiece = by_token ? ntok * nc8 : 0;
   auto piece_ptr = [&](int i) { return x + static_cast<int64_t>(i / nc8) * H + (i % nc8) * 8; };
   u32x4 xr[kPre];
   if (by_token) {
@@ -1252,10 +1263,9 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
   // gemm2_decode_kernel reads the pairs' slots from the workspace (the
   // activation-scale region, which the decode path does not use).
   if (blockIdx.x == 0 && wave == 0 && lane < npairs) reinterpret_cast<int32_t*>(work.acts)[lane] = slot_l;
-  const DecodeRoute rt = decode_route(slot_l, npairs);
+  const DecodeRoute rt = decode_route<ROWS>(slot_l, slots);
 
-  // The workgroup's subtile among all the step's, in slot order, and its
-  // column block; the grid bounds the subtiles (the same in every wave).
+  // The workgroup's subtile among all the step's and its column block; the grid bounds the subtiles (the same in every wave).
   const int ncb = static_cast<int>(I / 16);
   int gsi, cbk;
   xcd_item(ncb, gsi, cbk);
@@ -1266,9 +1276,23 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
   const int sub = gsi - __builtin_amdgcn_readlane(rt.start, lead);
   const unsigned long long mine = __ballot(slot_l == slot);
   const int count = __popcll(mine);
-  const int r0 = 16 * sub;  // below count
+  const int r0 = ROWS * sub;  // below count
   const int c0 = cbk * 16;
-  const int nrow = count - r0 < 16 ? count - r0 : 16;
+  const int nrow = count - r0 < ROWS ? count - r0 : ROWS;
+  // The subtile's rows: the slot's pairs in pair order, rows r0 .. r0 + nrow
+  // - 1; row r's pair goes to lane r (and lane 63 takes the other lanes').
+  const int rk = static_cast<int>(lane_prefix(mine)) - r0;
+  const bool in_sub = slot_l == slot && rk >= 0 && rk < ROWS;
+  const int row_pair = __builtin_amdgcn_ds_permute(4 * (in_sub ? rk : 63), lane);
+  if (!by_token) {
+    npiece = nrow * nc8;
+#pragma unroll
+    for (int i = 0; i < kPre; ++i) {
+      const int it = tid + kThreads * i < npiece ? tid + kThreads * i : 0;
+      const int r = it / nc8, p = __builtin_amdgcn_ds_bpermute(4 * r, row_pair);
+      xr[i] = *reinterpret_cast<const u32x4*>(x + static_cast<int64_t>(p / topk) * H + (it - r * nc8) * 8);
+    }
+  }
 
   // The slot's gate and up scales, then its weight rows, requested at once.
   const float* sg = w13_scale + (static_cast<int64_t>(slot) * (2 * I / kKB) + c0 / kKB) * KB;
@@ -1282,41 +1306,28 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
   KBlock c[kPerWave];
   load_chunk_b<kPerWave>(c, brow, kw0, KB);
 
-  // Token rows into LDS while the weights are in flight.
-  if (by_token) {
+  // Token rows into LDS while the weights are in flight: all of them, or the
+  // subtile's.
 #pragma unroll
-    for (int i = 0; i < kPre; ++i) {
-      const int it = tid + kThreads * i;
-      if (it < npiece) quant_piece(xr[i], it / nc8, (it % nc8) * 8);  // whole 16-lane groups
-    }
-    for (int it = tid + kThreads * kPre; it < npiece; it += kThreads)
-      quant_piece(*reinterpret_cast<const u32x4*>(piece_ptr(it)), it / nc8, (it % nc8) * 8);
+  for (int i = 0; i < kPre; ++i) {
+    const int it = tid + kThreads * i;
+    if (it < npiece) quant_piece(xr[i], it / nc8, (it % nc8) * 8);  // whole 16-lane groups
+  }
+  for (int it0 = kThreads * kPre; it0 < npiece; it0 += kThreads) {
+    const int it = it0 + tid < npiece ? it0 + tid : 0, r = it / nc8;
+    const int p = __builtin_amdgcn_ds_bpermute(4 * r, row_pair);
+    const int64_t t = by_token ? r : p / topk;
+    const u32x4 raw = *reinterpret_cast<const u32x4*>(x + t * H + (it - r * nc8) * 8);
+    if (it0 + tid < npiece) quant_piece(raw, r, (it - r * nc8) * 8);
   }
   if (tid < 2 * KB) s_sw[tid / KB][tid % KB] = sw;
-  // The subtile's rows: the slot's pairs in pair order, rows r0 .. r0 + 15;
-  // rows past nrow (outputs not stored) read the subtile's first row.
-  if (wave == 0) {
-    const int rk = static_cast<int>(lane_prefix(mine));
-    const bool in_sub = slot_l == slot && rk >= r0 && rk < r0 + 16;
-    const int lead_row = __ffsll(static_cast<long long>(__ballot(slot_l == slot && rk == r0))) - 1;
-    if (lane < 16) {
-      s_pair[lane] = -1;
-      s_arow[lane] = by_token ? lead_row / topk : 0;
-    }
-    if (in_sub) {
-      s_pair[rk - r0] = lane;
-      s_arow[rk - r0] = by_token ? lane / topk : rk - r0;
-    }
+  // Rows past nrow (outputs not stored) read the subtile's first row.
+  if (tid < 16) {
+    if (tid < ROWS) s_pair[tid] = tid < nrow ? row_pair : -1;
+    const int first = __builtin_amdgcn_readlane(row_pair, 0);
+    s_arow[tid] = by_token ? (tid < nrow ? row_pair : first) / topk : (tid < nrow ? tid : 0);
   }
   __syncthreads();  // s_aq, s_xs, s_sw, s_pair, s_arow
-  if (!by_token) {
-    for (int r = 0; r < nrow; ++r) {
-      const uint16_t* row = x + static_cast<int64_t>(s_pair[r] / topk) * H;
-      for (int c8 = tid * 8; c8 < H; c8 += kThreads * 8)
-        quant_piece(*reinterpret_cast<const u32x4*>(row + c8), r, c8);
-    }
-    __syncthreads();
-  }
 
   const uint8_t* arow = s_aq + s_arow[j] * H + 32 * q;
   auto load_a = [&](int kb0) {
@@ -1329,7 +1340,9 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
   };
   // Wave w scales and sums row 4q + w of the lane's 4-row group (gate and
   // up) in K order, one FMA per block, as gemm1_kernel does.
-  const int row = 4 * q + wave;
+  // The lanes past kLanes repeat the others'.
+  const int sl = lane & (kLanes - 1);
+  const int row = 4 * (sl >> 4) + wave;
   const int ar = s_arow[row];
   float acc_g = 0.f, acc_u = 0.f;
   for (int k0 = 0; k0 < KB; k0 += kSplitRound) {
@@ -1340,6 +1353,7 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
     for (int i = 0; i < kPerWave; ++i) {
       if (kw + i >= KB) continue;
       const f32x4 pg = mfma_k128(c[i].a, c[i].b[0]), pu = mfma_k128(c[i].a, c[i].b[1]);
+      if (lane >= kLanes) continue;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         s_part[wave * kPerWave + i][0][r][lane] = pg[r];
@@ -1350,12 +1364,12 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
     // Row `wave` of the lane's group: fixed offsets from one address, and
     // the whole round unrolled, so every LDS read of the sum is in flight
     // before the FMAs that consume it.
-    const float* sp = &s_part[0][0][wave][lane];
+    const float* sp = &s_part[0][0][wave][sl];
     const float* sx = s_xs + ar * KB + k0;
     auto sum_block = [&](int t) {
       const float sa = sx[t];
-      acc_g = fmaf(sp[(2 * t) * 256], sa * s_sw[0][k0 + t], acc_g);
-      acc_u = fmaf(sp[(2 * t + 1) * 256], sa * s_sw[1][k0 + t], acc_u);
+      acc_g = fmaf(sp[(2 * t) * 4 * kLanes], sa * s_sw[0][k0 + t], acc_g);
+      acc_u = fmaf(sp[(2 * t + 1) * 4 * kLanes], sa * s_sw[1][k0 + t], acc_u);
     };
     if (KB - k0 >= kSplitRound) {
 #pragma unroll
@@ -1373,10 +1387,10 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
     s_o[row * 16 + j] = static_cast<uint16_t>(bf16_bits(a));
   }
   __syncthreads();
-  if (tid < 16) {
+  if (tid < ROWS) {
     const int p = s_pair[tid];
     if (p >= 0) work.amax16[static_cast<int64_t>(p) * (I / 16) + c0 / 16] = s_m[tid];
-  } else if (tid < 48) {  // 16 rows x 2 pieces of 16 bytes
+  } else if (tid >= 16 && tid < 16 + 2 * ROWS) {  // ROWS rows x 2 pieces of 16 bytes
     const int rr = (tid - 16) >> 1, piece = tid & 1;
     const int p = s_pair[rr];
     if (p >= 0)
@@ -1385,22 +1399,28 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
   }
 }
 
-// gemm2 of a decode step with the top-k sum: one workgroup per (token, 8
-// output columns), so that a single token spreads its weight rows over 256
-// workgroups; lanes j and j + 8 of the MFMA operand read the same row (one
-// request), and columns 8-15 of the product are not used. Its waves take the token's pairs two at a time (wave w:
-// pairs w and w + 4, then w + 8 and w + 12, ...); each pair's 16 contributions are computed as
-// gemm2_narrow_kernel computes them (the token's quantised activation row as
-// every row of the MFMA operand, kNarrowChunk K blocks of weight rows per
-// load) and rounded to bf16; then the contributions are summed in k order
-// in fp32 and rounded once, as topk_sum_kernel does. A token's experts are
-// distinct slots, so its pairs share no weights. The pairs' slots come from
-// gemm1_decode_kernel's routing through the workspace, one load instead of
-// the ids and expert_map lookups. Pairs whose id is outside [0, E) add
-// nothing; so do pairs without a slot (the separate calls would read a
-// contribution never written). The slots, the routed weights and the first
-// activation pieces are requested first, then each wave's first two pairs'
-// weight rows, and the activations are quantised while those are in flight.
+// gemm2 of a decode step with the top-k sum: one workgroup per token and COLS
+// output columns. A single token takes 8, so that its weight rows spread over
+// 256 workgroups at H = 2048; then lanes j and j + 8 of the MFMA operand read
+// the same row (one request), and columns 8-15 of the product are not used.
+// More tokens fill the GPU with 16 columns, and half as many workgroups
+// quantise each token's activations (4 tokens, 32 experts 2048 x 512: 13.1 ->
+// 9.2 us; the quantisation was the larger part of a workgroup's
+// instructions). Its waves take the token's pairs two at a time (wave w:
+// pairs w and w + 4, then w + 8 and w + 12, ...); each pair's contributions
+// are computed as gemm2_narrow_kernel computes them (the token's quantised
+// activation row as every row of the MFMA operand, kNarrowChunk K blocks of
+// weight rows per load) and rounded to bf16; then the contributions are
+// summed in k order in fp32 and rounded once, as topk_sum_kernel does. A
+// token's experts are distinct slots, so its pairs share no weights. The
+// pairs' slots come from gemm1_decode_kernel's routing through the workspace,
+// one load instead of the ids and expert_map lookups. Pairs whose id is
+// outside [0, E) add nothing; so do pairs without a slot (the separate calls
+// would read a contribution never written). The slots, the routed weights and
+// the first activation pieces are requested first, then each wave's first two
+// pairs' weight rows, and the activations are quantised while those are in
+// flight.
+template <int COLS>
 __global__ void __launch_bounds__(kThreads) gemm2_decode_kernel(
     int64_t H, int64_t I, int topk, const float* __restrict__ topk_weight, const uint8_t* __restrict__ w2,
     const float* __restrict__ w2_scale, Work work, uint16_t* __restrict__ out) {
@@ -1409,11 +1429,11 @@ __global__ void __launch_bounds__(kThreads) gemm2_decode_kernel(
   extern __shared__ __attribute__((aligned(16))) uint8_t s_act[];  // [topk][I] fp8 activations
   __shared__ int s_slot[kDecodePairs];
   __shared__ float s_as[kDecodePairs * 4];  // activation scales [pair][K block], K blocks of a round
-  __shared__ uint16_t s_c[kDecodePairs][kDecodeCols2];
+  __shared__ uint16_t s_c[kDecodePairs][COLS];
 
-  const int ncol = static_cast<int>(H / kDecodeCols2);
+  const int ncol = static_cast<int>(H / COLS);
   const int t = static_cast<int>(blockIdx.x) / ncol;
-  const int n0 = (static_cast<int>(blockIdx.x) - t * ncol) * kDecodeCols2;
+  const int n0 = (static_cast<int>(blockIdx.x) - t * ncol) * COLS;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int q = lane >> 4, j = lane & 15;
   const int KB = static_cast<int>(I / kKB);
@@ -1452,10 +1472,10 @@ __global__ void __launch_bounds__(kThreads) gemm2_decode_kernel(
     am[i][1] = *reinterpret_cast<const u32x4*>(m + 4);
   }
 
-  // A pair's weight rows for output columns n0 .. n0 + 7 and their scales.
+  // A pair's weight rows for output columns n0 .. n0 + COLS - 1 and their scales.
   auto pair_rows = [&](int slot, const uint8_t*& brow, const float*& sw) {
     const int sl = slot < 0 ? 0 : slot;
-    brow = w2 + static_cast<int64_t>(sl) * H * I + static_cast<int64_t>(n0 + (j & (kDecodeCols2 - 1))) * I + 32 * q;
+    brow = w2 + static_cast<int64_t>(sl) * H * I + static_cast<int64_t>(n0 + (j & (COLS - 1))) * I + 32 * q;
     sw = w2_scale + (static_cast<int64_t>(sl) * (H / kKB) + n0 / kKB) * KB;
   };
   // A chunk's weight rows of two pairs, with their K blocks' scales.
@@ -1576,7 +1596,7 @@ __global__ void __launch_bounds__(kThreads) gemm2_decode_kernel(
   auto finish = [&](const int (&kk)[2], const int (&slot)[2], const float (&acc)[2], const float (&tw)[2]) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      if (kk[h] >= topk || q != 0 || j >= kDecodeCols2) continue;
+      if (kk[h] >= topk || q != 0 || j >= COLS) continue;
       s_c[kk[h]][j] = slot[h] < 0 ? 0 : static_cast<uint16_t>(bf16_bits(acc[h] * tw[h]));
     }
   };
@@ -1616,7 +1636,7 @@ __global__ void __launch_bounds__(kThreads) gemm2_decode_kernel(
     finish(kk, slot, acc, tw);
   }
   __syncthreads();
-  if (tid < kDecodeCols2) {
+  if (tid < COLS) {
     // The token's contributions in k order, eight LDS reads in flight at a
     // time.
     float sum = 0.f;
@@ -2392,28 +2412,34 @@ int xp_moe_decode_experts(const uint16_t* x, int64_t T, int64_t H, const void* t
   XP_REQUIRE(work_bytes >= need, "%s: workspace of %lld B, needs %lld", what, (long long)work_bytes, (long long)need);
   Work w;
   work_layout(npairs, I, &w, static_cast<uint8_t*>(work));
-  // One workgroup per 16-row subtile of an occupied slot and 16 columns.
-  // The subtiles number at most min(npairs, slots), plus npairs / 16 when a
-  // slot can hold more than 16 pairs (sum over slots of ceil(c / 16) with
-  // the counts c summing to npairs).
-  const int64_t subs = (npairs < slots ? npairs : slots) + (npairs > 16 ? npairs / 16 : 0);
+  // One workgroup per subtile of an occupied slot and 16 columns: 4 or 8 rows
+  // where that many tokens cannot fill more of a slot, else 16. With m slots
+  // occupied by n pairs, sum over slots of ceil(c / rows) is at most
+  // m + (n - m) / rows, which grows with m up to min(n, slots).
+  const int rows = T <= 4 ? 4 : T <= 8 ? 8 : 16;
+  const int64_t occupied = npairs < slots ? npairs : slots;
+  const int64_t subs = occupied + (npairs - occupied) / rows;
   const int64_t subs8 = (subs + 7) / 8 * 8;  // the XCD-aware grid covers whole groups of 8
   const dim3 g1(static_cast<unsigned>(subs8 * (I / 16)));
+  const size_t lds = static_cast<size_t>(rows) * static_cast<size_t>(H);
+  auto gate_up = [&](auto act_c) {
+    constexpr int ACT = decltype(act_c)::value;
+    auto* kernel = rows == 4 ? gemm1_decode_kernel<ACT, 4> : rows == 8 ? gemm1_decode_kernel<ACT, 8>
+                                                                       : gemm1_decode_kernel<ACT, 16>;
+    hipLaunchKernelGGL(kernel, g1, dim3(kThreads), lds, as_stream(stream), x, H, I, topk_ids, topk_elem_bytes,
+                       static_cast<int>(npairs), static_cast<int>(topk), expert_map, pair_slot,
+                       static_cast<int>(num_experts), static_cast<int>(slots), w13, w13_scale, w);
+  };
   if (activation == XP_ACT_GELU)
-    hipLaunchKernelGGL(gemm1_decode_kernel<XP_ACT_GELU>, g1, dim3(kThreads), static_cast<size_t>(16 * H),
-                       as_stream(stream), x, H, I, topk_ids, topk_elem_bytes, static_cast<int>(npairs),
-                       static_cast<int>(topk), expert_map, pair_slot, static_cast<int>(num_experts),
-                       static_cast<int>(slots), w13, w13_scale, w);
+    gate_up(Int<XP_ACT_GELU>{});
   else
-    hipLaunchKernelGGL(gemm1_decode_kernel<XP_ACT_SILU>, g1, dim3(kThreads), static_cast<size_t>(16 * H),
-                       as_stream(stream), x, H, I, topk_ids, topk_elem_bytes, static_cast<int>(npairs),
-                       static_cast<int>(topk), expert_map, pair_slot, static_cast<int>(num_experts),
-                       static_cast<int>(slots), w13, w13_scale, w);
+    gate_up(Int<XP_ACT_SILU>{});
   int rc = check_launch("gemm1_decode_kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL(gemm2_decode_kernel, dim3(static_cast<unsigned>(T * (H / kDecodeCols2))), dim3(kThreads),
-                     static_cast<size_t>(topk * I), as_stream(stream), H, I, static_cast<int>(topk), topk_weight,
-                     w2, w2_scale, w, out);
+  const int cols = T == 1 ? 8 : 16;
+  hipLaunchKernelGGL(cols == 8 ? gemm2_decode_kernel<8> : gemm2_decode_kernel<16>,
+                     dim3(static_cast<unsigned>(T * (H / cols))), dim3(kThreads), static_cast<size_t>(topk * I),
+                     as_stream(stream), H, I, static_cast<int>(topk), topk_weight, w2, w2_scale, w, out);
   return check_launch("gemm2_decode_kernel");
 }
 

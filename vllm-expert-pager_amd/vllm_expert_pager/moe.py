@@ -232,13 +232,16 @@ def topk_sum(contrib: torch.Tensor, topk_ids: torch.Tensor, num_experts: int,
 DECODE_PAIRS = 64  # a fused decode call's limits: pairs (T * topk), H, topk * I
 DECODE_MAX_H = 4096
 DECODE_ACT_BYTES = 32768
-# Above this many pairs the separate calls are faster than the fused step:
-# the down projection of the fused step reads each pair's w2 rows once per
-# token, while run_experts reads an expert's rows once for all its tokens.
-# Measured with 2048 x 512 experts at top-8: 4 tokens 38 us fused against
-# 46 us separate, 5 tokens 48 against 50, 6 tokens 58 against 52, 8 tokens
-# 81 against 47.
+# Above these many pairs or tokens the step takes the separate calls: the
+# down projection of the fused step reads each pair's w2 rows once per token,
+# while run_experts reads an expert's rows once for all its tokens. Measured,
+# us per layer in a graph, fused against separate: 256 experts 2048 x 512 at
+# top-8: 4 tokens 26 against 43, 5 tokens 31 against 46, 8 tokens 41 against
+# 44; 64 experts 2048 x 768 at top-8: 5 tokens 38 against 55, 8 tokens 56
+# against 54; 16 experts 4096 x 1024 at top-2: 8 tokens 42 against 50, 12
+# tokens 64 against 55, 16 tokens 79 against 55.
 DECODE_STEP_PAIRS = 40
+DECODE_STEP_TOKENS = 8
 
 
 def decode_fits(x: torch.Tensor, topk_ids: torch.Tensor, intermediate: int) -> bool:
@@ -251,7 +254,8 @@ def decode_fits(x: torch.Tensor, topk_ids: torch.Tensor, intermediate: int) -> b
 def decode_pays(x: torch.Tensor, topk_ids: torch.Tensor, intermediate: int) -> bool:
     """Whether a decode step takes ``decode_experts`` (else the separate calls)."""
     T, topk = _shape(topk_ids)
-    return T * topk <= DECODE_STEP_PAIRS and decode_fits(x, topk_ids, intermediate)
+    return (T <= DECODE_STEP_TOKENS and T * topk <= DECODE_STEP_PAIRS
+            and decode_fits(x, topk_ids, intermediate))
 
 
 def decode_experts(

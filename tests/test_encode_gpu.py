@@ -65,6 +65,15 @@ def test_matches_host_encoder_group_counts(groups):
     _matches_host_encoder("realistic", 64, groups)
 
 
+# Few groups with chunks of at least 512 values: eight waves share each pair of
+# groups. Odd group counts leave a spare half-wave; codes of 1 bit and of 9 put
+# the segments' starts in, at the ends of and early loads across the words.
+@pytest.mark.parametrize("dist", ["realistic", "uniform", "constant", "long_codes", "one_symbol_rare"])
+@pytest.mark.parametrize("chunk, groups", [(512, 1), (512, 5), (1024, 3)])
+def test_matches_host_encoder_segments(dist, chunk, groups):
+    _matches_host_encoder(dist, chunk, groups)
+
+
 def _matches_host_encoder(dist, chunk, groups):
     codec = _codec()
     n = groups * chunk * 32

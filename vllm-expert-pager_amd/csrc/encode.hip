@@ -10,7 +10,8 @@
 //      whenever fewer than LIMIT bits are left, so a chunk whose last symbol
 //      starts at bit b needs (b + LIMIT - 1) / 32 + 1 words; summed per
 //      group and scanned into gstart, written to the record's header.
-// encode_groups_kernel, one workgroup per 8 groups of a row:
+// encode_groups_kernel, one workgroup per 8 groups of a row (per 2 where the
+// groups are few, see kSegments):
 //   4. the code again, from the row's LUT (every symbol has a code of at
 //      most LIMIT bits, so each one appears in the 9-bit table with its
 //      length, and the canonical codes follow from the lengths); then each
@@ -407,10 +408,32 @@ __global__ void __launch_bounds__(kPlanThreads) encode_plan_kernel(EncodeArgs a)
   for (int64_t i = nbytes / 4 + tid; i < a.pitch / 4; i += kPlanThreads) reinterpret_cast<uint32_t*>(rec)[i] = 0;
 }
 
+// Waves that share a group's chunks, each a segment of all of them, where the
+// groups are few. A chain of 512 symbols takes a wave 48 us however few
+// groups there are; the state at a segment's start follows from the code
+// lengths before it: a lane's bit position P is their sum, the words it has
+// loaded number (P(last symbol) + LIMIT - 1) / 32 + 1, and a group's are the
+// sum over its lanes. A word loaded early belongs to a symbol at most 8 before
+// the start, so a wave walks those 8 without writing; the word that a start
+// falls into is joined from both waves' bits in LDS (a segment has at least 64
+// bits, so it ends in the next wave's).
+// The sums and the 8 symbols are a quarter more work, so rows that fill the
+// chip keep one wave for two whole groups. The whole call, without the check,
+// for 1, 16, 32 and 64 rows of 128 groups: 67, 84, 106 and 161 us with one
+// segment, 37, 66, 107 and 170 with four, 31, 61, 94 and 160 with eight.
+constexpr int kSegments = 8;
+constexpr int kMinSegment = 64;  // symbols: a block of loads
+constexpr int64_t kSegmentGroups = 4096;
+
 // SPLIT: the words per group come from encode_words_kernel; the workgroup
 // sums those before its groups and writes its part of gstart and of the tail.
-template <bool SPLIT>
-__global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, int blocks_per_row) {
+// SEG > 1: two groups per workgroup, cut into SEG segments.
+template <bool SPLIT, int SEG>
+__global__ void __launch_bounds__(SEG > 1 ? 64 * SEG : 256) encode_groups_kernel(EncodeArgs a, int blocks_per_row) {
+  constexpr int kThreads = SEG > 1 ? 64 * SEG : xp::kThreads;
+  constexpr int kGroupsPerBlock = SEG > 1 ? 2 : xp::kGroupsPerBlock;
+  __shared__ uint32_t s_bits[SEG][64];  // SEG > 1: a lane's bits in each segment
+  __shared__ uint32_t s_head[SEG][64];  // SEG > 1: the segment's bits of the word that its start falls into
   __shared__ int32_t s_len[code::kSyms];
   __shared__ uint32_t s_code[code::kSyms];  // code | length << 16
   __shared__ uint2 s_pair[code::kSyms * code::kSyms];  // see encode_pair
@@ -486,8 +509,8 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
     if (tid < code::kSyms) s_code[tid] = static_cast<uint32_t>(code) | (static_cast<uint32_t>(length) << 16);
   }
   __syncthreads();
-  static_assert(kThreads == code::kSyms * code::kSyms, "a thread per pair of symbols");
-  {
+  static_assert(kThreads >= code::kSyms * code::kSyms, "a thread per pair of symbols");
+  if (tid < code::kSyms * code::kSyms) {
     const uint32_t first = s_code[tid & 15], second = s_code[tid >> 4];
     const uint32_t l0 = first >> 16, l01 = l0 + (second >> 16);
     s_pair[tid] = make_uint2((first & 0xffffu) | ((second & 0xffffu) << l0), (l0 << 26) | l01);
@@ -503,13 +526,15 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
   const int mwords = chunk / 8;
   const uint32_t total = static_cast<uint32_t>(s_gstart[kGroupsPerBlock]);  // every word position is below it
   {
-    const int g0 = gfirst + 2 * wave;
-    if (g0 >= G) return;
+    const int pair_of_groups = SEG > 1 ? 0 : wave, seg = SEG > 1 ? wave : 0;
+    const int g0 = gfirst + 2 * pair_of_groups;
+    if (g0 >= G) return;  // SEG > 1: never
     const int g = g0 + (upper ? 1 : 0);
     const bool live = g < G;  // a spare half-wave walks the last group and writes nothing
     const int gg = live ? g : G - 1;
-    const uint8_t* src = raw + (int64_t(gg) * XP_LANES + li) * chunk;
-    uint32_t* fx = fixed + int64_t(gg) * mwords * XP_LANES + li;
+    const int length = chunk / SEG, begin = seg * length;  // of the wave's segment
+    const uint8_t* src = raw + (int64_t(gg) * XP_LANES + li) * chunk + begin;
+    uint32_t* fx = fixed + (int64_t(gg) * mwords + begin / 8) * XP_LANES + li;
     // Word positions within each half's group, both below 2^16 (a group's
     // words are at most 32 chunks of 9-bit codes), packed in one scalar
     // register: the lower half's in bits 0-15, the upper half's in 16-31
@@ -517,10 +542,10 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
     // half's refills of a symbol (at most 32) never borrows. A lane's word
     // positions are relative; gbase makes them absolute.
     constexpr uint32_t kBias = 64;
-    const uint32_t gs_lo = static_cast<uint32_t>(s_gstart[2 * wave]);
-    const uint32_t gs_hi = static_cast<uint32_t>(s_gstart[2 * wave + (g0 + 1 < G ? 1 : 0)]);
+    const uint32_t gs_lo = static_cast<uint32_t>(s_gstart[2 * pair_of_groups]);
+    const uint32_t gs_hi = static_cast<uint32_t>(s_gstart[2 * pair_of_groups + (g0 + 1 < G ? 1 : 0)]);
     const uint32_t gbase = upper ? gs_hi - kBias : gs_lo;
-    const uint32_t limit = live ? total : 0u;
+    uint32_t limit = live ? total : 0u;
     uint32_t offs = kBias << 16;
     // The decoder has fewer than LIMIT bits left before the symbol that starts
     // at bit P of the lane's stream exactly when the words it has loaded
@@ -533,6 +558,7 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
     uint32_t Qp = Q ^ 0x80000000u;              // of the symbol before (bits below 26 are not used)
     uint32_t acc = 0, accbits = 0;              // the bits of the word being filled
     uint32_t wcur = 0, wprev = 0;               // positions of the last word loaded and the one before
+    bool head = false;                          // the next word complete is the one that the segment starts in
     // Two symbols at a time (`at` is 8 x (second * 16 + first)): a pair's
     // entry holds both codes in a row, their length l01 in bits 0-5 and the
     // first's in bits 26-31. Loads are at least three symbols apart (a load
@@ -545,7 +571,7 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
     // The loop is VALU bound: about 20 instructions a symbol, half of what
     // symbol by symbol with a two-entry queue of loaded words took. 256 rows
     // of 2 MiB: 485 -> 358 us (2.2 TB/s read and written); one row, a chain of
-    // 512 symbols in 64 waves, 71 -> 48 us. Reading a 16-byte piece's eight
+    // 512 symbols in 64 waves, 71 -> 48 us (in segments, see kSegments, 12). Reading a 16-byte piece's eight
     // entries ahead of its pairs changed neither.
     auto encode_pair = [&](uint32_t at) {
       const uint2 t = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(s_pair) + at);
@@ -573,7 +599,12 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
       if (full) {
         const bool alone = (q1 & 0x7C000000u) == 0x7C000000u;
         const uint32_t at_word = gbase + (alone ? wcur : wprev);
-        if (at_word < limit) huff[at_word] = word;
+        if (SEG > 1 && head) {
+          s_head[seg][lane] = word;
+          head = false;
+        } else if (at_word < limit) {
+          huff[at_word] = word;
+        }
       }
       acc = full ? static_cast<uint32_t>(shifted >> 32) : word;
       accbits = bits & 31u;
@@ -581,13 +612,56 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
     // A lane's values in blocks of 64 (four 16-byte loads back to back, so
     // each cache line of its chunk is fetched about twice instead of once
     // per 16 values), the next block loaded while this one is encoded.
-    const int nv = chunk < 64 ? chunk / 16 : 4;  // loads per block
+    const int nv = SEG == 1 && chunk < 64 ? chunk / 16 : 4;  // loads per block
     u32x4 cur[4], nxt[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (j < nv) cur[j] = *reinterpret_cast<const u32x4*>(src + 16 * j);
-    for (int i0 = 0; i0 < chunk; i0 += 16 * nv) {
-      if (i0 + 16 * nv < chunk) {
+    if constexpr (SEG > 1) {
+      // The 16 values before the segment (the first segment: its own).
+      const u32x4 pre = *reinterpret_cast<const u32x4*>(src - (seg > 0 ? 16 : 0));
+      uint32_t lb[4];
+      pack_lengths(s_len, lb);
+      uint32_t bits = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        bits += sum_lengths4(cur[j].x, lb) + sum_lengths4(cur[j].y, lb) + sum_lengths4(cur[j].z, lb) +
+                sum_lengths4(cur[j].w, lb);
+      for (int i = 64; i < length; i += 16) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(src + i);
+        bits += sum_lengths4(v.x, lb) + sum_lengths4(v.y, lb) + sum_lengths4(v.z, lb) + sum_lengths4(v.w, lb);
+      }
+      s_bits[seg][lane] = bits;
+      __syncthreads();
+      uint32_t start = 0;
+#pragma unroll
+      for (int k = 0; k < SEG - 1; ++k) start += k < seg ? s_bits[k][lane] : 0u;
+      if (seg > 0) {
+        const uint32_t p8 = start - sum_lengths4(pre.z, lb) - sum_lengths4(pre.w, lb);  // of the 8th symbol before
+        const uint32_t p9 = p8 - static_cast<uint32_t>(s_len[pre.y >> 27 & 15u]);
+        Q = (p8 + XP_LIMIT - 1) << 26;
+        Qp = (p9 + XP_LIMIT - 1) << 26;
+        uint32_t loaded = (p9 + XP_LIMIT - 1) / 32 + 1;
+#pragma unroll
+        for (int d = 16; d >= 1; d >>= 1) loaded += __shfl_xor(loaded, d, 32);
+        offs = static_cast<uint32_t>(__builtin_amdgcn_readlane(loaded, 0)) +
+               ((static_cast<uint32_t>(__builtin_amdgcn_readlane(loaded, 32)) + kBias) << 16);
+        accbits = p8 & 31u;
+        const uint32_t to = limit;
+        limit = 0;  // nothing is written
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const uint32_t ex = (k ? pre.w : pre.z) & 0x78787878u, z = ex | (ex >> 4);
+          encode_pair(z & 0x7F8u);
+          encode_pair((z >> 16) & 0x7F8u);
+        }
+        limit = to;
+        acc = 0;
+        head = accbits != 0;
+      }
+    }
+    for (int i0 = 0; i0 < length; i0 += 16 * nv) {
+      if (i0 + 16 * nv < length) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           if (j < nv) nxt[j] = *reinterpret_cast<const u32x4*>(src + i0 + 16 * nv + 16 * j);
@@ -623,6 +697,14 @@ __global__ void __launch_bounds__(kThreads) encode_groups_kernel(EncodeArgs a, i
     // started at or after bit 1 - LIMIT = -8 of it, and the next one, all
     // zeros, if it started at or after bit 24.
     const int last = static_cast<int>(accbits) - static_cast<int>((Q - (Qp & 0xFC000000u)) >> 26);
+    if constexpr (SEG > 1) {
+      __syncthreads();
+      if (seg < SEG - 1) {  // the next segment's start is in the word being filled, unless a word ends there
+        const uint32_t at_word = gbase + (last >= 24 ? wprev : wcur);
+        if (accbits != 0 && at_word < limit) huff[at_word] = acc | s_head[seg + 1][lane];
+        return;
+      }
+    }
     if (last >= 24) {
       if (gbase + wprev < limit) huff[gbase + wprev] = acc;
       if (gbase + wcur < limit) huff[gbase + wcur] = 0;
@@ -681,7 +763,7 @@ int xp_encode_rows_split(const uint8_t* raw, int64_t rows, int64_t raw_stride, i
     hipLaunchKernelGGL(encode_plan_kernel, dim3(static_cast<unsigned>(rows)), dim3(kPlanThreads), 0,
                        as_stream(stream), a);
     if (int rc = check_launch("encode_plan_kernel")) return rc;
-    hipLaunchKernelGGL(encode_groups_kernel<false>, grid, dim3(kThreads), 0, as_stream(stream), a,
+    hipLaunchKernelGGL((encode_groups_kernel<false, 1>), grid, dim3(kThreads), 0, as_stream(stream), a,
                        static_cast<int>(blocks));
     return check_launch("encode_groups_kernel");
   }
@@ -706,8 +788,14 @@ int xp_encode_rows_split(const uint8_t* raw, int64_t rows, int64_t raw_stride, i
   hipLaunchKernelGGL(encode_words_kernel, dim3(static_cast<unsigned>(rows * word_blocks)), dim3(kThreads), 0,
                      as_stream(stream), a, static_cast<int>(groups), static_cast<int>(word_blocks));
   if (int rc = check_launch("encode_words_kernel")) return rc;
-  hipLaunchKernelGGL(encode_groups_kernel<true>, grid, dim3(kThreads), 0, as_stream(stream), a,
-                     static_cast<int>(blocks));
+  if (rows * G <= kSegmentGroups && chunk >= kSegments * kMinSegment) {
+    const int64_t pairs = (G + 1) / 2;
+    hipLaunchKernelGGL((encode_groups_kernel<true, kSegments>), dim3(static_cast<unsigned>(rows * pairs)),
+                       dim3(64 * kSegments), 0, as_stream(stream), a, static_cast<int>(pairs));
+  } else {
+    hipLaunchKernelGGL((encode_groups_kernel<true, 1>), grid, dim3(kThreads), 0, as_stream(stream), a,
+                       static_cast<int>(blocks));
+  }
   return check_launch("encode_groups_kernel");
 }
 

@@ -137,10 +137,12 @@ def test_encode_of_a_gpu_row():
 
 # The plan by several workgroups per row against the one by a workgroup per
 # row: rows of 1, 2, 4 and 8 groups per counting workgroup (up to 2048
-# workgroups take one group each), more than one 64 KiB part per row, and rows
+# workgroups take one group each), more than one 64 KiB part per row, chunks that
+# are counted (from 512 values, with a partial last part and more groups than a
+# workgroup takes at once), and rows
 # that do not fit, whose records stay as they were.
 @pytest.mark.parametrize("count, groups, chunk", [(1, 1, 16), (1, 130, 64), (300, 9, 16), (700, 11, 16),
-                                                  (1500, 17, 16), (3, 40, 1024)])
+                                                  (1500, 17, 16), (3, 40, 1024), (2, 5, 512), (300, 9, 512), (5, 9, 1024)])
 def test_split_plan_equals_a_workgroup_per_row(count, groups, chunk):
     from vllm_expert_pager import _native as nat
 

@@ -2,8 +2,8 @@
 // (encode, codec.py:125-198), producing the bytes of the host encoder
 // (codec_host.cpp) and of the reference.
 //
-// The plan: encode_hist_kernel and encode_words_kernel, several workgroups
-// per row, or without a workspace encode_plan_kernel, one per row:
+// The plan: encode_hist_kernel and encode_words_kernel (chunks of 512 values
+// and more: encode_count_kernel and encode_sizes_kernel), several workgroups per row, or without a workspace encode_plan_kernel, one per row:
 //   1. exponent histogram: per-thread counters in LDS, then summed;
 //   2. the code by one wave, the 512-entry LUT by the workgroup;
 //   3. Huffman words per chunk: the decoder loads a word before symbol i
@@ -41,6 +41,7 @@ constexpr int kPlanThreads = 1024;
 constexpr int kPlanUnroll = 4;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 struct EncodeArgs {
   const uint8_t* raw;
@@ -56,6 +57,7 @@ struct EncodeArgs {
   uint32_t* hist;      // split plan: [row][part][16] exponent counts
   int32_t* words;      // split plan: [row][G] Huffman words per group
   int parts;           // split plan: parts of a row's histogram
+  uint32_t* counts;    // split plan, long chunks: [row][chunk][8] (see encode_count_kernel)
 };
 
 // A row's code, built by one wave and the same in every lane of it: lane l
@@ -205,7 +207,8 @@ __device__ __forceinline__ void write_lut(const int32_t* s_len, const int32_t* s
 // parts of the rows, so that a few rows fill the GPU and many rows leave no
 // partly empty round of one workgroup per row. One 2 MiB row: 266 us in one
 // workgroup, 7 + 12 us here; 256 rows: 316 us, 111 + 142 us (537 MB read
-// twice, at 4.8 and 3.8 TB/s; half of what was saved is the code's).
+// twice, at 4.8 and 3.8 TB/s; half of what was saved is the code's). Long
+// chunks are read once, see encode_count_kernel.
 
 // Exponent counts of part `blockIdx.x % parts` (kPartBytes values) of a row.
 // Each thread counts into its own LDS counters with atomic adds whose result
@@ -249,7 +252,24 @@ __global__ void __launch_bounds__(kThreads) encode_hist_kernel(EncodeArgs a) {
   if (at == 0) a.hist[static_cast<int64_t>(blockIdx.x) * code::kSyms + sym] = t;
 }
 
-// The row's code from its parts' counts (each workgroup for itself; the
+// The row's code from its parts' counts, by the first wave of a workgroup.
+__device__ __forceinline__ void wave_row_code(const EncodeArgs& a, int row, int32_t* s_len, int32_t* s_code) {
+  const int tid = threadIdx.x;
+  const uint32_t* h = a.hist + static_cast<int64_t>(row) * a.parts * code::kSyms + (tid & 15);
+  uint32_t t = 0;
+#pragma unroll 4
+  for (int i = tid >> 4; i < a.parts; i += 4) t += h[i * code::kSyms];
+  t += __shfl_xor(t, 16, 64);
+  t += __shfl_xor(t, 32, 64);
+  const int length = wave_code_lengths(t);
+  const int code = wave_canonical_code(length);
+  if (tid < code::kSyms) {
+    s_len[tid] = length;
+    s_code[tid] = code;
+  }
+}
+
+// The row's code (each workgroup for itself; the
 // row's first one writes the LUT), then the Huffman words of `groups` groups
 // (1 to 8: as few as leave the launch within kWordsBlocks workgroups, so that
 // a row's code is not built many more times than there are groups in flight).
@@ -271,18 +291,7 @@ __global__ void __launch_bounds__(kThreads) encode_words_kernel(EncodeArgs a, in
   for (int u = 0; u < kPlanUnroll; ++u)
     if (lo + tid * 16 + u * kStep < hi) v[u] = *reinterpret_cast<const u32x4*>(raw + lo + tid * 16 + u * kStep);
   if (tid < 64) {
-    const uint32_t* h = a.hist + static_cast<int64_t>(row) * a.parts * code::kSyms + (tid & 15);
-    uint32_t t = 0;
-#pragma unroll 4
-    for (int i = tid >> 4; i < a.parts; i += 4) t += h[i * code::kSyms];
-    t += __shfl_xor(t, 16, 64);
-    t += __shfl_xor(t, 32, 64);
-    const int length = wave_code_lengths(t);
-    const int code = wave_canonical_code(length);
-    if (tid < code::kSyms) {
-      s_len[tid] = length;
-      s_code[tid] = code;
-    }
+    wave_row_code(a, row, s_len, s_code);
   } else if (tid < 64 + kGroupsPerBlock) {
     s_words[tid - 64] = 0;
   }
@@ -304,6 +313,124 @@ __global__ void __launch_bounds__(kThreads) encode_words_kernel(EncodeArgs a, in
   }
   __syncthreads();
   if (tid < groups && g0 + tid < a.G) a.words[static_cast<int64_t>(row) * a.G + g0 + tid] = s_words[tid];
+}
+
+// ---- the same for long chunks, whose values are read once ----
+//
+// A chunk's words follow from its exponent counts and its last symbol, 32
+// bytes for 512 values or more, so the histogram launch leaves those (an
+// eighth more work: 119 -> 131 us for 256 rows of 2 MiB, 4.3 TB/s) and the
+// second launch reads them instead of the row (143 -> 19 us, the code's build
+// for most of it). One row: 6 + 12 -> 7 + 9 us. Chunks below 512 values would
+// write and read back more than an eighth of the row, and keep the two passes.
+
+constexpr int kCountChunk = 512;  // values per chunk from which a row's chunks are counted
+
+// encode_hist_kernel with each chunk's counts: word s of a chunk holds symbol
+// s's count in bits 0-15 and symbol s + 8's in bits 16-27, word 7 the
+// chunk's last symbol in bits 28-31. A wave takes 8 chunks at a time, 8 lanes
+// each, so that a load covers whole lines; the lanes' counters run on over the
+// chunks, and a chunk's counts are what its lanes' sum grew by. Each lane sums
+// two symbols, its eight reads rotated by the symbol so that they hit 64 banks.
+__global__ void __launch_bounds__(kThreads) encode_count_kernel(EncodeArgs a) {
+  __shared__ uint32_t s_hist[code::kSyms][kThreads];
+  const int row = blockIdx.x / a.parts, part = blockIdx.x % a.parts;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c8 = lane >> 3, l8 = lane & 7;
+  const int64_t lo = part * kPartBytes, hi = lo + kPartBytes < a.n ? lo + kPartBytes : a.n;
+  const int chunk = a.chunk;
+  // A row is whole groups of 32 chunks, and a part whole sets of 8.
+  const int sets = static_cast<int>((hi - lo) / (8 * chunk));
+  const uint8_t* src = a.raw + static_cast<int64_t>(row) * a.raw_stride + lo + c8 * chunk + 16 * l8;
+  uint32_t* out = a.counts + (static_cast<int64_t>(row) * (a.n / chunk) + lo / chunk) * 8;
+  u32x4 v[4];
+  auto request = [&](int set, int at) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const u32x4*>(src + int64_t(set) * 8 * chunk + at + 128 * k);
+  };
+  if (wave < sets) request(wave, 0);
+  for (int s = 0; s < code::kSyms; ++s) s_hist[s][tid] = 0;
+  uint32_t below0 = 0, below1 = 0;  // the sums after the set before
+  for (int set = wave; set < sets; set += kThreads / 64) {
+    uint32_t last = 0;
+    for (int at = 0; at < chunk; at += kCountChunk) {
+      u32x4 x[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[k] = v[k];
+      if (at + kCountChunk < chunk)
+        request(set, at + kCountChunk);
+      else if (set + kThreads / 64 < sets)
+        request(set + kThreads / 64, 0);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t w[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int b = 0; b < 4; ++b) atomicAdd(&s_hist[(w[i] >> (8 * b + 3)) & 15u][tid], 1u);
+      }
+      last = x[3].w >> 27 & 15u;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    uint32_t sum0 = 0, sum1 = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int at = (tid & ~7) + ((i + l8) & 7);
+      sum0 += s_hist[l8][at];
+      sum1 += s_hist[l8 + 8][at];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint32_t n0 = sum0 - below0, n1 = sum1 - below1;
+    below0 = sum0;
+    below1 = sum1;
+    out[(int64_t(set) * 8 + c8) * 8 + l8] = n0 | n1 << 16 | (l8 == 7 ? last << 28 : 0u);
+  }
+  __syncthreads();
+  const int sym = tid >> 4, at = tid & 15;
+  uint32_t t = 0;
+#pragma unroll
+  for (int i = 0; i < kThreads / 16; ++i) t += s_hist[sym][at + 16 * i];
+#pragma unroll
+  for (int d = 8; d >= 1; d >>= 1) t += __shfl_xor(t, d, 16);
+  if (at == 0) a.hist[static_cast<int64_t>(blockIdx.x) * code::kSyms + sym] = t;
+}
+
+// encode_words_kernel from the chunks' counts, a thread per chunk, `groups`
+// (a multiple of 8) groups per workgroup.
+__global__ void __launch_bounds__(kThreads) encode_sizes_kernel(EncodeArgs a, int groups, int blocks_per_row) {
+  __shared__ int32_t s_len[code::kSyms];
+  __shared__ int32_t s_code[code::kSyms];
+  const int row = blockIdx.x / blocks_per_row, part = blockIdx.x % blocks_per_row;
+  const int tid = threadIdx.x;
+  const int g0 = part * groups, g1 = g0 + groups < a.G ? g0 + groups : a.G;
+  const uint32_t* counts = a.counts + static_cast<int64_t>(row) * (a.n / a.chunk) * 8;
+  int c = g0 * XP_LANES + tid;
+  u32x4 lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
+  if (c < g1 * XP_LANES) {
+    lo = *reinterpret_cast<const u32x4_any*>(counts + int64_t(c) * 8);
+    hi = *reinterpret_cast<const u32x4_any*>(counts + int64_t(c) * 8 + 4);
+  }
+  if (tid < 64) wave_row_code(a, row, s_len, s_code);
+  __syncthreads();
+  if (part == 0) write_lut(s_len, s_code, a.lut + static_cast<int64_t>(row) * a.lut_stride, kThreads);
+  uint32_t len[code::kSyms];
+#pragma unroll
+  for (int s = 0; s < code::kSyms; ++s) len[s] = static_cast<uint32_t>(s_len[s]);
+  while (c < g1 * XP_LANES) {  // the same for all lanes of a half-wave
+    const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    uint32_t bits = 0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) bits += (w[s] & 0xffffu) * len[s] + ((w[s] >> 16) & 0x0fffu) * len[s + 8];
+    bits -= static_cast<uint32_t>(s_len[w[7] >> 28]);  // not the last symbol
+    uint32_t words = (bits + XP_LIMIT - 1) / 32 + 1;
+#pragma unroll
+    for (int d = 16; d >= 1; d >>= 1) words += __shfl_xor(words, d, 32);
+    if ((tid & 31) == 0) a.words[static_cast<int64_t>(row) * a.G + c / XP_LANES] = static_cast<int32_t>(words);
+    c += kThreads;
+    if (c < g1 * XP_LANES) {
+      lo = *reinterpret_cast<const u32x4_any*>(counts + int64_t(c) * 8);
+      hi = *reinterpret_cast<const u32x4_any*>(counts + int64_t(c) * 8 + 4);
+    }
+  }
 }
 
 // ---- the plan of a row by one workgroup ----
@@ -420,7 +547,8 @@ __global__ void __launch_bounds__(kPlanThreads) encode_plan_kernel(EncodeArgs a)
 // The sums and the 8 symbols are a quarter more work, so rows that fill the
 // chip keep one wave for two whole groups. The whole call, without the check,
 // for 1, 16, 32 and 64 rows of 128 groups: 67, 84, 106 and 161 us with one
-// segment, 37, 66, 107 and 170 with four, 31, 61, 94 and 160 with eight.
+// segment, 37, 66, 107 and 170 with four, 31, 61, 94 and 160 with eight (with
+// the plan's second pass over the rows still in them).
 constexpr int kSegments = 8;
 constexpr int kMinSegment = 64;  // symbols: a block of loads
 constexpr int64_t kSegmentGroups = 4096;
@@ -571,7 +699,7 @@ __global__ void __launch_bounds__(SEG > 1 ? 64 * SEG : 256) encode_groups_kernel
     // The loop is VALU bound: about 20 instructions a symbol, half of what
     // symbol by symbol with a two-entry queue of loaded words took. 256 rows
     // of 2 MiB: 485 -> 358 us (2.2 TB/s read and written); one row, a chain of
-    // 512 symbols in 64 waves, 71 -> 48 us (in segments, see kSegments, 12). Reading a 16-byte piece's eight
+    // 512 symbols in 64 waves, 71 -> 48 us (in segments, see kSegments, 13). Reading a 16-byte piece's eight
     // entries ahead of its pairs changed neither.
     auto encode_pair = [&](uint32_t at) {
       const uint2 t = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(s_pair) + at);
@@ -725,7 +853,8 @@ extern "C" {
 
 int64_t xp_encode_workspace_bytes(int64_t rows, int64_t n, int64_t chunk) {
   if (rows <= 0 || n <= 0 || chunk <= 0) return 0;
-  return 4 * rows * (hist_parts(n) * code::kSyms + n / (chunk * XP_LANES));
+  return 4 * rows *
+         (hist_parts(n) * code::kSyms + n / (chunk * XP_LANES) + (chunk >= kCountChunk ? n / chunk * 8 : 0));
 }
 
 int xp_encode_rows(const uint8_t* raw, int64_t rows, int64_t raw_stride, int64_t n, int64_t chunk, uint8_t* records,
@@ -755,7 +884,7 @@ int xp_encode_rows_split(const uint8_t* raw, int64_t rows, int64_t raw_stride, i
              "xp_encode_rows: pitch %lld is not a positive multiple of 16", (long long)pitch);
   XP_REQUIRE(lut_stride >= XP_LUT_BYTES, "xp_encode_rows: lut_stride=%lld", (long long)lut_stride);
   EncodeArgs a{raw, raw_stride, n, static_cast<int>(chunk), static_cast<int>(G), records, pitch,
-               luts, lut_stride, needed, nullptr, nullptr, 0};
+               luts, lut_stride, needed, nullptr, nullptr, 0, nullptr};
   const int64_t blocks = (G + kGroupsPerBlock - 1) / kGroupsPerBlock;
   XP_REQUIRE(rows * blocks <= INT32_MAX, "xp_encode_rows: %lld rows x %lld blocks", (long long)rows, (long long)blocks);
   const dim3 grid(static_cast<unsigned>(rows * blocks));
@@ -777,16 +906,28 @@ int xp_encode_rows_split(const uint8_t* raw, int64_t rows, int64_t raw_stride, i
   a.parts = static_cast<int>(parts);
   a.hist = static_cast<uint32_t*>(work);
   a.words = static_cast<int32_t*>(work) + rows * parts * code::kSyms;
-  hipLaunchKernelGGL(encode_hist_kernel, dim3(static_cast<unsigned>(rows * parts)), dim3(kThreads), 0,
-                     as_stream(stream), a);
+  a.counts = reinterpret_cast<uint32_t*>(a.words + rows * G);
+  const bool counted = chunk >= kCountChunk;
+  const dim3 plan_grid(static_cast<unsigned>(rows * parts));
+  if (counted)
+    hipLaunchKernelGGL(encode_count_kernel, plan_grid, dim3(kThreads), 0, as_stream(stream), a);
+  else
+    hipLaunchKernelGGL(encode_hist_kernel, plan_grid, dim3(kThreads), 0, as_stream(stream), a);
   if (int rc = check_launch("encode_hist_kernel")) return rc;
-  int64_t groups = 1;
-  while (groups < kGroupsPerBlock && rows * ((G + groups - 1) / groups) > kWordsBlocks) groups *= 2;
+  // Counted chunks: a workgroup's threads take 8 groups at once.
+  int64_t groups = counted ? kGroupsPerBlock : 1;
+  while (groups < (counted ? kMaxGroups : kGroupsPerBlock) && rows * ((G + groups - 1) / groups) > kWordsBlocks)
+    groups *= 2;
   const int64_t word_blocks = (G + groups - 1) / groups;
   XP_REQUIRE(rows * word_blocks <= INT32_MAX, "xp_encode_rows_split: %lld rows x %lld blocks", (long long)rows,
              (long long)word_blocks);
-  hipLaunchKernelGGL(encode_words_kernel, dim3(static_cast<unsigned>(rows * word_blocks)), dim3(kThreads), 0,
-                     as_stream(stream), a, static_cast<int>(groups), static_cast<int>(word_blocks));
+  const dim3 words_grid(static_cast<unsigned>(rows * word_blocks));
+  if (counted)
+    hipLaunchKernelGGL(encode_sizes_kernel, words_grid, dim3(kThreads), 0, as_stream(stream), a,
+                       static_cast<int>(groups), static_cast<int>(word_blocks));
+  else
+    hipLaunchKernelGGL(encode_words_kernel, words_grid, dim3(kThreads), 0, as_stream(stream), a,
+                       static_cast<int>(groups), static_cast<int>(word_blocks));
   if (int rc = check_launch("encode_words_kernel")) return rc;
   if (rows * G <= kSegmentGroups && chunk >= kSegments * kMinSegment) {
     const int64_t pairs = (G + 1) / 2;

@@ -120,6 +120,34 @@ def test_quant_tokens_bit_exact():
 
 # 5000 x 8 pairs: each of the 16 waves walks 2500 pairs, in batches of 1024
 # (the last one partial).
+def test_quant_tokens_of_every_maximum():
+    """Groups whose maxima are all the finite bf16 magnitudes, their other values spread
+    below (signed zeros and subnormals among them), give the codes of a division by the
+    scale; where the maximum is infinite, finite values give zeros of their sign and
+    infinite ones the code of a clamped NaN."""
+    moe = _moe()
+    rng = np.random.default_rng(5)
+    amax = np.arange(0x7F80, dtype=np.int64).reshape(-1, 1)
+    bits = (rng.random((0x7F80, 128)) ** 4 * (amax + 1)).astype(np.int64)  # at most the maximum
+    near = rng.integers(0, 1600, (0x7F80, 128))  # half within the 12 octaves that fp8 resolves
+    bits = np.where(rng.random(bits.shape) < 0.5, np.maximum(amax - near, 0), bits)
+    bits[:, 7:8] = amax
+    bits[:, 8] = 0
+    bits |= rng.integers(0, 2, bits.shape) << 15
+    x = torch.from_numpy(bits.astype(np.uint16).view(np.int16).reshape(-1, 4096)).cuda().view(torch.bfloat16)
+    xq, xs = moe.quant_tokens(x)
+    q, s = M.quant_groups(x.float().cpu().numpy())
+    np.testing.assert_array_equal(xs.cpu().numpy(), s)
+    np.testing.assert_array_equal(xq.view(torch.uint8).cpu().numpy(), q)
+    inf = x[-1:].clone()
+    inf[0, ::128] = float("inf")
+    inf[0, 1::128] = float("-inf")
+    code = moe.quant_tokens(inf)[0].view(torch.uint8)[0].cpu().numpy().reshape(-1, 128)
+    assert (code[:, :2] == 0xFE).all()
+    sign = (inf[0].view(torch.int16).cpu().numpy().reshape(-1, 128) < 0)[:, 2:]
+    np.testing.assert_array_equal(code[:, 2:], np.where(sign, 0x80, 0))
+
+
 @pytest.mark.parametrize("T, topk, E, slots", [(50, 4, 20, 12), (300, 4, 6, 6), (1, 8, 64, 32), (5000, 8, 256, 200)])
 def test_route_lists_mapped_pairs(T, topk, E, slots):
     moe = _moe()

@@ -64,14 +64,47 @@ __device__ __forceinline__ uint32_t bf16_bits(float v) {
 
 __device__ __forceinline__ float bf16_value(uint32_t u16) { return __uint_as_float(u16 << 16); }
 
-// fp32 -> fp8 e4m3 (OCP), round to nearest even; callers clamp to +-448.
-__device__ __forceinline__ uint32_t to_fp8(float v) {
-  return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(v, v, 0, false)) & 0xffu;
-}
-
 __device__ __forceinline__ float quant_scale(float amax) { return fmaxf(amax, kEps) / kFp8Max; }
 
 __device__ __forceinline__ float clamp_fp8(float v) { return fminf(fmaxf(v, -kFp8Max), kFp8Max); }
+
+// Quantisation by one scale s: fp8(clamp(v / s)), e4m3 (OCP), to nearest even.
+// The quotient is v * (1 / s) with one step of its remainder, three
+// instructions where a division takes about ten and a quarter-rate one: v / s
+// rounded correctly, as 1 / s is (Markstein 1990), where the remainder is
+// exact. For a bf16 value and the scale of a bf16 maximum it is, except where
+// both forms are below 2^-10, which rounds to zero of the same sign (all
+// 32641 maxima with all values up to them, infinities among them, compared on
+// the CPU). The remainder is taken as q * s - v, which keeps -0, and an
+// infinite scale enters it as 0: finite values become 0, infinite ones NaN,
+// as they do by division. Layers of 256 experts 2048 x 512: 1 token 14.0 -> 13.7
+// us, 2048 tokens 254 -> 250, 8192 tokens 577 -> 566.
+struct Quant {
+  float inv, fin;
+  __device__ __forceinline__ explicit Quant(float s) : inv(1.0f / s), fin(s < INFINITY ? s : 0.0f) {}
+  __device__ __forceinline__ float operator()(float v) const {
+    const float q = v * inv;
+    return clamp_fp8(fmaf(-fmaf(q, fin, -v), inv, q));
+  }
+};
+
+// Four quantised values as bytes, the first lowest.
+__device__ __forceinline__ uint32_t fp8x4(float a, float b, float c, float d) {
+  return static_cast<uint32_t>(
+      __builtin_amdgcn_cvt_pk_fp8_f32(c, d, __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false), true));
+}
+
+// Eight bf16 values (two per word) quantised.
+__device__ __forceinline__ uint2 quant_words(const u32x4& raw, float s) {
+  const Quant q(s);
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[2 * i] = q(bf16_value(raw[i] & 0xffffu));
+    v[2 * i + 1] = q(bf16_value(raw[i] >> 16));
+  }
+  return make_uint2(fp8x4(v[0], v[1], v[2], v[3]), fp8x4(v[4], v[5], v[6], v[7]));
+}
 
 // a = bf16(bf16(act(g)) * u) for bf16 values g (gate) and u (up): the
 // activation in fp32 as vLLM's activation kernels compute it, returned in
@@ -148,13 +181,7 @@ __device__ __forceinline__ void quant_token(const uint16_t* __restrict__ x, int6
     for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
     amax = row16_max(amax);
     const float s = quant_scale(amax);
-    uint32_t q0 = 0, q1 = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      q0 |= to_fp8(clamp_fp8(v[i] / s)) << (8 * i);
-      q1 |= to_fp8(clamp_fp8(v[4 + i] / s)) << (8 * i);
-    }
-    *reinterpret_cast<uint2*>(xq + t * H + c0) = make_uint2(q0, q1);
+    *reinterpret_cast<uint2*>(xq + t * H + c0) = quant_words(raw, s);
     if ((tid & 15) == 0) xs[t * (H / kKB) + c0 / kKB] = s;
   }
 }
@@ -930,10 +957,8 @@ __global__ void __launch_bounds__(kGemmWaves * 64) gemm1_kernel(const uint8_t* _
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi) {
         const int row = 16 * mi + j;
-        const float sc = s_q[row];
-        uint32_t w = 0;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) w |= to_fp8(clamp_fp8(acc[mi][0][r] / sc)) << (8 * r);
+        const Quant qr(s_q[row]);
+        const uint32_t w = fp8x4(qr(acc[mi][0][0]), qr(acc[mi][0][1]), qr(acc[mi][0][2]), qr(acc[mi][0][3]));
         *reinterpret_cast<uint32_t*>(stg + row * kRowB + ((wave ^ (row & 7)) << 4) + 4 * q) = w;
       }
     });
@@ -1230,13 +1255,7 @@ __global__ void __launch_bounds__(kThreads) gemm1_decode_kernel(
     for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
     amax = row16_max(amax);
     const float sc = quant_scale(amax);
-    uint32_t q0 = 0, q1 = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      q0 |= to_fp8(clamp_fp8(v[i] / sc)) << (8 * i);
-      q1 |= to_fp8(clamp_fp8(v[4 + i] / sc)) << (8 * i);
-    }
-    *reinterpret_cast<uint2*>(s_aq + r * H + c8) = make_uint2(q0, q1);
+    *reinterpret_cast<uint2*>(s_aq + r * H + c8) = quant_words(raw, sc);
     if ((tid & 15) == 0) s_xs[r * KB + c8 / kKB] = sc;
   };
   // With one or two tokens, all their rows are requested before the routing
@@ -1515,15 +1534,7 @@ __global__ void __launch_bounds__(kThreads) gemm2_decode_kernel(
     for (int u = 0; u < 4; ++u) mx = fmaxf(mx, __uint_as_float(mm[1][u]));
     const float sc = quant_scale(mx);
     if (c8 % kKB == 0 && g < 4) s_as[k * 4 + g] = sc;
-    uint32_t q0 = 0, q1 = 0;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      q0 |= to_fp8(clamp_fp8(bf16_value(v[u] & 0xffffu) / sc)) << (16 * u);
-      q0 |= to_fp8(clamp_fp8(bf16_value(v[u] >> 16) / sc)) << (16 * u + 8);
-      q1 |= to_fp8(clamp_fp8(bf16_value(v[2 + u] & 0xffffu) / sc)) << (16 * u);
-      q1 |= to_fp8(clamp_fp8(bf16_value(v[2 + u] >> 16) / sc)) << (16 * u + 8);
-    }
-    *reinterpret_cast<uint2*>(s_act + k * I + c8) = make_uint2(q0, q1);
+    *reinterpret_cast<uint2*>(s_act + k * I + c8) = quant_words(v, sc);
   };
   if (tid < topk) s_slot[tid] = my_slot;
 #pragma unroll
@@ -1727,15 +1738,7 @@ __global__ void __launch_bounds__(kThreads) gemm2_narrow_kernel(int64_t H, int64
       for (int k = 1; k < 8; ++k) mx = fmaxf(mx, m[k]);
       const float sc = quant_scale(mx);
       if (c8 % kKB == 0) s_as[r * KB + g] = sc;
-      uint32_t q0 = 0, q1 = 0;
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        q0 |= to_fp8(clamp_fp8(bf16_value(v[k] & 0xffffu) / sc)) << (16 * k);
-        q0 |= to_fp8(clamp_fp8(bf16_value(v[k] >> 16) / sc)) << (16 * k + 8);
-        q1 |= to_fp8(clamp_fp8(bf16_value(v[2 + k] & 0xffffu) / sc)) << (16 * k);
-        q1 |= to_fp8(clamp_fp8(bf16_value(v[2 + k] >> 16) / sc)) << (16 * k + 8);
-      }
-      *reinterpret_cast<uint2*>(s_act + r * kQuantK + c8) = make_uint2(q0, q1);
+      *reinterpret_cast<uint2*>(s_act + r * kQuantK + c8) = quant_words(v, sc);
     }
     __syncthreads();  // s_act, s_as (and s_w, s_sw)
     for (int kc = 0; kc < nk; kc += CH) {

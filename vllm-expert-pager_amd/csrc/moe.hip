@@ -625,9 +625,15 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t off, void* dst)
       : "v"(off), "s"(uniform_ptr(base)), "s"(__builtin_amdgcn_readfirstlane(lds_addr(dst)))
       : "memory");
 }
-// dma16 marked non-temporal, for weight rows: each is read once per launch,
-// so they should not push the activation rows (re-read by every column block
-// of a tile) out of the caches. 3-4% off the prefill GEMMs.
+// dma16 marked non-temporal, for weight rows that are read once per launch:
+// they should not push the activation rows (re-read by every column block of a
+// tile) out of the caches. Where experts have several tiles, each reads the
+// rows again, and marked rows are no longer in its L2: dma_weights<false>.
+// Whole layers of 2048 x 512 experts, marked and not: 23 tokens (4 layers) 287
+// and 305 us, 333 tokens 97 and 101, 2048 tokens (64 pairs per expert) 246 and
+// 244, 8192 tokens (256) 566 and 533. So the line is a mean of one whole tile
+// (stream_weights). Chosen per item, by a branch around the loads, it cost the
+// small calls 20%.
 __device__ __forceinline__ void dma16_stream(const void* base, uint32_t off, void* dst) {
   uint32_t saved;
   asm volatile(
@@ -636,6 +642,14 @@ __device__ __forceinline__ void dma16_stream(const void* base, uint32_t off, voi
       : "v"(off), "s"(uniform_ptr(base)), "s"(__builtin_amdgcn_readfirstlane(lds_addr(dst)))
       : "memory");
 }
+template <bool STREAM>
+__device__ __forceinline__ void dma_weights(const void* base, uint32_t off, void* dst) {
+  if constexpr (STREAM)
+    dma16_stream(base, off, dst);
+  else
+    dma16(base, off, dst);
+}
+inline bool stream_weights(int64_t npairs, int64_t slots) { return npairs < slots * kWM; }
 __device__ __forceinline__ void dma4(const void* base, uint32_t off, void* dst) {
   uint32_t saved;
   asm volatile(
@@ -752,7 +766,7 @@ __device__ __forceinline__ AOffsets a_offsets(const int* s_row, int64_t lda, int
 // workgroup width or the tile height. Then a = bf16(bf16(silu(bf16 gate)) *
 // bf16 up) is quantised to fp8 per row over the workgroup's 128 columns, one
 // scale group. Only the 16-row subtiles that hold pairs are multiplied.
-template <int ACT>
+template <int ACT, bool STREAM>
 __global__ void __launch_bounds__(kGemmWaves * 64) gemm1_kernel(const uint8_t* __restrict__ xq,
                                                                const float* __restrict__ xs, int64_t H, int64_t I,
                                                                int topk, const uint8_t* __restrict__ w13,
@@ -810,7 +824,7 @@ __global__ void __launch_bounds__(kGemmWaves * 64) gemm1_kernel(const uint8_t* _
   auto issue = [&](int stage, const uint8_t* wb, const AOffsets& ao, int kb, int nmi) {
     const uint8_t* bsrc = wb + kb * kRowB;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dma16_stream(bsrc, boff[i], s_b[stage] + (32 * wave + 8 * i) * kRowB);
+    for (int i = 0; i < 4; ++i) dma_weights<STREAM>(bsrc, boff[i], s_b[stage] + (32 * wave + 8 * i) * kRowB);
     int ops = 4;
     if (wave < nmi) {
       const uint8_t* asrc = xq + kb * kRowB;
@@ -1786,7 +1800,7 @@ __global__ void __launch_bounds__(kThreads) gemm2_narrow_kernel(int64_t H, int64
 // waves owns 16 TB columns and runs the K blocks in order over the tile's
 // fp8 activations; persistent over items through the operand ring as
 // gemm1_kernel.
-template <int TB>
+template <int TB, bool STREAM>
 __global__ void __launch_bounds__(kGemmWaves * 64) gemm2_kernel(int64_t H, int64_t I,
                                                                const float* __restrict__ topk_weight,
                                                                const uint8_t* __restrict__ w2,
@@ -1841,7 +1855,7 @@ __global__ void __launch_bounds__(kGemmWaves * 64) gemm2_kernel(int64_t H, int64
   auto issue = [&](int stage, const uint8_t* wb, const AOffsets& ao, int kb, int nmi) {
     const uint8_t* bsrc = wb + kb * kRowB;
 #pragma unroll
-    for (int i = 0; i < 2 * TB; ++i) dma16_stream(bsrc, boff[i], s_b[stage] + (16 * TB * wave + 8 * i) * kRowB);
+    for (int i = 0; i < 2 * TB; ++i) dma_weights<STREAM>(bsrc, boff[i], s_b[stage] + (16 * TB * wave + 8 * i) * kRowB);
     int ops = 2 * TB;
     if (wave < nmi) {
       const uint8_t* asrc = work.act + kb * kRowB;
@@ -2215,26 +2229,21 @@ int launch_experts(const uint8_t* xq, const float* xs, int64_t T, int64_t topk, 
     const int64_t per_xcd_tiles = (wmax + 7) / 8;  // wide tiles of one XCD, at most
     // One workgroup per CU: the operand ring takes most of its LDS.
     const int64_t n1 = std::min<int64_t>(per_xcd, per_xcd_tiles * (I / (16 * kGemmWaves)));
-    if (act == XP_ACT_GELU)
-      hipLaunchKernelGGL(gemm1_kernel<XP_ACT_GELU>, dim3(static_cast<unsigned>(8 * n1)), dim3(64 * kGemmWaves), 0,
-                         as_stream(stream), xq, xs, H, I, static_cast<int>(topk), w13, w13_scale, pairs, wide, wmax,
-                         npairs, w);
-    else
-      hipLaunchKernelGGL(gemm1_kernel<XP_ACT_SILU>, dim3(static_cast<unsigned>(8 * n1)), dim3(64 * kGemmWaves), 0,
-                         as_stream(stream), xq, xs, H, I, static_cast<int>(topk), w13, w13_scale, pairs, wide, wmax,
-                         npairs, w);
+    const bool stream_w = stream_weights(npairs, slots);
+    auto* gemm1 = act == XP_ACT_GELU
+                      ? (stream_w ? gemm1_kernel<XP_ACT_GELU, true> : gemm1_kernel<XP_ACT_GELU, false>)
+                      : (stream_w ? gemm1_kernel<XP_ACT_SILU, true> : gemm1_kernel<XP_ACT_SILU, false>);
+    hipLaunchKernelGGL(gemm1, dim3(static_cast<unsigned>(8 * n1)), dim3(64 * kGemmWaves), 0, as_stream(stream), xq, xs,
+                       H, I, static_cast<int>(topk), w13, w13_scale, pairs, wide, wmax, npairs, w);
     rc = check_launch("gemm1_kernel");
     if (rc) return rc;
     // 256 output columns per item where H allows, else 128.
-    if (H % (2 * kBN) == 0) {
-      const int64_t n2 = std::min<int64_t>(per_xcd, per_xcd_tiles * (H / (2 * kBN)));
-      hipLaunchKernelGGL(gemm2_kernel<2>, dim3(static_cast<unsigned>(8 * n2)), dim3(64 * kGemmWaves), 0,
-                         as_stream(stream), H, I, topk_weight, w2, w2_scale, pairs, wide, wmax, npairs, w, out);
-    } else {
-      const int64_t n2 = std::min<int64_t>(per_xcd, per_xcd_tiles * (H / kBN));
-      hipLaunchKernelGGL(gemm2_kernel<1>, dim3(static_cast<unsigned>(8 * n2)), dim3(64 * kGemmWaves), 0,
-                         as_stream(stream), H, I, topk_weight, w2, w2_scale, pairs, wide, wmax, npairs, w, out);
-    }
+    const int tb = H % (2 * kBN) == 0 ? 2 : 1;
+    const int64_t n2 = std::min<int64_t>(per_xcd, per_xcd_tiles * (H / (tb * kBN)));
+    auto* gemm2 = tb == 2 ? (stream_w ? gemm2_kernel<2, true> : gemm2_kernel<2, false>)
+                          : (stream_w ? gemm2_kernel<1, true> : gemm2_kernel<1, false>);
+    hipLaunchKernelGGL(gemm2, dim3(static_cast<unsigned>(8 * n2)), dim3(64 * kGemmWaves), 0, as_stream(stream), H, I,
+                       topk_weight, w2, w2_scale, pairs, wide, wmax, npairs, w, out);
     return check_launch("gemm2_kernel");
   }
   const int64_t tiles8 = (bound + 7) / 8 * 8;  // the XCD-aware grids cover whole groups of 8 tiles

@@ -313,9 +313,10 @@ int xp_encode_rows(const uint8_t* raw, int64_t rows, int64_t raw_stride,
                    void* stream);
 
 /* xp_encode_rows with a workspace (xp_encode_workspace_bytes bytes, device
- * memory, no initial contents), in which several workgroups plan a row: the
- * faster form for any number of rows, many times so for a few. Same bytes;
- * a null `work` is xp_encode_rows. */
+ * memory, no initial contents; 0 for sizes that xp_encode_rows refuses), in
+ * which several workgroups plan a row: the faster form for any number of
+ * rows, many times so for a few. Same bytes; a null `work` is
+ * xp_encode_rows. */
 int64_t xp_encode_workspace_bytes(int64_t rows, int64_t n, int64_t chunk);
 int xp_encode_rows_split(const uint8_t* raw, int64_t rows, int64_t raw_stride,
                          int64_t n, int64_t chunk, uint8_t* records,

@@ -1,4 +1,4 @@
-"""Argument checks of the decode launchers, on the CPU (no kernel is launched).
+"""Argument checks of the decode and encode launchers, on the CPU (no kernel is launched).
 
 ``decode_rows`` and ``decode_rows_from_ram`` write row r of ``dst[i]`` at
 ``r * shape[1] * element_size`` bytes from the tensor's start, so every
@@ -41,3 +41,22 @@ def test_dst_rows_must_be_contiguous_2d(monkeypatch, bad):
     scale = [torch.zeros((4, 2), dtype=torch.float32)]
     with pytest.raises(ValueError, match=r"dst\[0\] must be a contiguous 2-D tensor"):
         codec.decode_rows_from_ram(idx, idx, idx, idx, 0, staging, dst, lut, scale, scale)
+
+
+@pytest.mark.parametrize("chunk", [0, -512, 8, 2048, 1 << 58, 1 << 59, 1 << 62, (1 << 63) - 1])
+def test_encode_refuses_any_chunk_size(monkeypatch, chunk):
+    """Chunks outside 16..1024 are a ValueError, also where chunk * 32 overflows 64 bits (to 0
+    at 2^59, by which the workspace's size was divided)."""
+    monkeypatch.setattr(codec.nat, "require_device", lambda t, what: None)
+    monkeypatch.setattr(codec.nat, "stream", lambda: None)
+    assert codec.nat.lib().xp_encode_workspace_bytes(1, 1 << 20, chunk) == 0
+    with pytest.raises(ValueError, match="chunk="):
+        codec.encode_rows(torch.zeros((1, 1 << 14), dtype=torch.uint8), 16, chunk)
+
+
+def test_encode_workspace_of_refused_rows():
+    """No rows, too many, and rows of no group or of more than the encoder takes need no workspace."""
+    size = codec.nat.lib().xp_encode_workspace_bytes
+    assert size(3, 128 * 16384, 512) == 3 * 4 * (32 * 16 + 128 + 4096 * 8)
+    assert size(1, 16383, 512) == size(0, 1 << 20, 512) == size(-1, 1 << 20, 512) == size(1, -(1 << 20), 512) == 0
+    assert size(1 << 31, 1 << 20, 512) == size(1, 1 << 62, 512) == 0

@@ -852,9 +852,11 @@ using namespace xp;
 extern "C" {
 
 int64_t xp_encode_workspace_bytes(int64_t rows, int64_t n, int64_t chunk) {
-  if (rows <= 0 || n <= 0 || chunk <= 0) return 0;
-  return 4 * rows *
-         (hist_parts(n) * code::kSyms + n / (chunk * XP_LANES) + (chunk >= kCountChunk ? n / chunk * 8 : 0));
+  // Sizes that the encoder refuses need nothing, and must not overflow here.
+  if (rows <= 0 || rows > INT32_MAX || chunk < 16 || chunk > 1024) return 0;
+  const int64_t G = n / (chunk * XP_LANES);
+  if (G < 1 || G > kMaxGroups) return 0;
+  return 4 * rows * (hist_parts(n) * code::kSyms + G + (chunk >= kCountChunk ? n / chunk * 8 : 0));
 }
 
 int xp_encode_rows(const uint8_t* raw, int64_t rows, int64_t raw_stride, int64_t n, int64_t chunk, uint8_t* records,

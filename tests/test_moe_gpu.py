@@ -550,3 +550,22 @@ def test_decode_rows_by_token_count(T, topk, E, route):
     want = _separate(moe, xb, tw_t, ids_t, emap, E, E, w)
     got = moe.decode_experts(xb, tw_t, ids_t, emap, E, *w, E)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# Steps of more than 8 tokens with few experts per token, which take the fused
+# launches: 16 rows per gate/up workgroup, from the smallest experts to the
+# widest rows of which two workgroups share a CU's LDS, and 40 tokens of one
+# pair each.
+@pytest.mark.parametrize("T, topk, E, H, I", [(9, 1, 12, 512, 128), (40, 1, 300, 512, 128), (20, 2, 7, 1024, 256),
+                                              (24, 1, 16, 2688, 384), (10, 4, 16, 2048, 512)])
+def test_decode_steps_of_many_tokens(T, topk, E, H, I):
+    moe = _moe()
+    x, tw, ids, w13, w13s, w2, w2s = _case(T + E, E, H, I, T, topk)
+    xb, emap = _bf16(x), torch.arange(E, dtype=torch.int32, device="cuda").flip(0).contiguous()
+    tw_t, ids_t, *w = _dev(tw, ids, w13, w13s, w2, w2s)
+    assert moe.decode_pays(xb, ids_t, I)
+    want = _separate(moe, xb, tw_t, ids_t, emap, E, E, w)
+    pair_slot = emap[ids_t.long()].flatten().contiguous()
+    for slots in (None, pair_slot):
+        got = moe.decode_experts(xb, tw_t, ids_t, emap, E, *w, E, pair_slot=slots)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))

@@ -232,16 +232,30 @@ def topk_sum(contrib: torch.Tensor, topk_ids: torch.Tensor, num_experts: int,
 DECODE_PAIRS = 64  # a fused decode call's limits: pairs (T * topk), H, topk * I
 DECODE_MAX_H = 4096
 DECODE_ACT_BYTES = 32768
-# Above these many pairs or tokens the step takes the separate calls: the
-# down projection of the fused step reads each pair's w2 rows once per token,
-# while run_experts reads an expert's rows once for all its tokens. Measured,
-# us per layer in a graph, fused against separate: 256 experts 2048 x 512 at
-# top-8: 4 tokens 26 against 43, 5 tokens 31 against 46, 8 tokens 41 against
-# 44; 64 experts 2048 x 768 at top-8: 5 tokens 38 against 55, 8 tokens 56
-# against 54; 16 experts 4096 x 1024 at top-2: 8 tokens 42 against 50, 12
-# tokens 64 against 55, 16 tokens 79 against 55.
+# The pager's choice between the fused step and the separate calls. The down
+# projection of the fused step reads each pair's w2 rows once per token and
+# quantises a token's activations in each of its H / 16 workgroups, while
+# run_experts reads an expert's rows once for all its tokens. Measured, us per
+# layer in a graph, six layers of their own weights in turn, fused against
+# separate:
+# - Pairs: between 40 and 64 either may win (8 tokens at top-8: 256 experts
+#   2048 x 512 41 against 44, 64 experts 2048 x 768 56 against 54).
+# - Up to 8 tokens a gate/up workgroup takes 4 or 8 rows, and the fused step
+#   wins up to 40 pairs (16 experts 4096 x 1024 at top-2, 8 tokens: 45 against
+#   53) but for the largest experts at top-4 (62 against 59).
+# - With more tokens it takes 16 rows of H columns in LDS: two workgroups share
+#   a CU up to H = 2688. Above, nothing is gained (3072 x 1024 at top-2, 9
+#   tokens: 55 against 53; 4096 x 512 at top-4, 9 tokens: 49 against 47).
+# - Below, T * H bounds the quantising workgroups (2048 x 128 at top-1: 32
+#   tokens 21 against 26, 40 tokens 24 against 24) and T * H * I the rows read
+#   again (2688 x 384 at top-1: 24 tokens 38 against 39, 32 tokens 43 against
+#   40; 2048 x 1024: 12 tokens 26 against 35). Small experts gain most: 9
+#   tokens at top-1, 512 x 128: 10 against 19, 2048 x 512: 14 against 23.
 DECODE_STEP_PAIRS = 40
 DECODE_STEP_TOKENS = 8
+DECODE_WIDE_MAX_H = 2688
+DECODE_WIDE_COLS = 1 << 16  # T * H
+DECODE_WIDE_BYTES = 3 << 23  # T * H * I
 
 
 def decode_fits(x: torch.Tensor, topk_ids: torch.Tensor, intermediate: int) -> bool:
@@ -254,8 +268,11 @@ def decode_fits(x: torch.Tensor, topk_ids: torch.Tensor, intermediate: int) -> b
 def decode_pays(x: torch.Tensor, topk_ids: torch.Tensor, intermediate: int) -> bool:
     """Whether a decode step takes ``decode_experts`` (else the separate calls)."""
     T, topk = _shape(topk_ids)
-    return (T <= DECODE_STEP_TOKENS and T * topk <= DECODE_STEP_PAIRS
-            and decode_fits(x, topk_ids, intermediate))
+    if T * topk > DECODE_STEP_PAIRS or not decode_fits(x, topk_ids, intermediate):
+        return False
+    H = x.shape[1]
+    return T <= DECODE_STEP_TOKENS or (H <= DECODE_WIDE_MAX_H and T * H <= DECODE_WIDE_COLS
+                                       and T * H * intermediate <= DECODE_WIDE_BYTES)
 
 
 def decode_experts(

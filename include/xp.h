@@ -445,6 +445,20 @@ int xp_moe_experts(const uint8_t* xq, const float* xs, int64_t T,
                    const int32_t* tiles, void* work, int64_t work_bytes,
                    uint16_t* out, int activation, void* stream);
 
+/* xp_moe_experts over a slab that holds a part of the experts (a chunk of
+ * them): num_experts is the count that xp_moe_route was given. Same results
+ * and bits; the T*topk pairs are then taken to be spread over num_experts
+ * experts rather than `slots`, which decides whether the prefill kernels keep
+ * weight rows in the caches (128 pairs per expert and more). */
+int xp_moe_experts_part(const uint8_t* xq, const float* xs, int64_t T,
+                        int64_t topk, const float* topk_weight, int64_t H,
+                        int64_t I, const uint8_t* w13, const float* w13_scale,
+                        const uint8_t* w2, const float* w2_scale,
+                        int64_t slots, int64_t num_experts,
+                        const int32_t* offsets, const int32_t* pairs,
+                        const int32_t* tiles, void* work, int64_t work_bytes,
+                        uint16_t* out, int activation, void* stream);
+
 /* Workspace bytes xp_moe_experts_noalloc holds per device (32 MiB: a
  * 2048-token top-8 prefill at I = 512 needs 27.5 MB). */
 #define XP_MOE_SCRATCH_BYTES (32LL << 20)

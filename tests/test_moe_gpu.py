@@ -569,3 +569,36 @@ def test_decode_steps_of_many_tokens(T, topk, E, H, I):
     for slots in (None, pair_slot):
         got = moe.decode_experts(xb, tw_t, ids_t, emap, E, *w, E, pair_slot=slots)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# The prefill GEMMs' second template argument tells whether weight rows are
+# marked as read once: up to a mean of 128 pairs per expert, over the experts
+# that the map covers. A chunk's slab holds 8 of 64 experts here, so that 4096
+# pairs are 64 per expert and 8192 are 128.
+@pytest.mark.parametrize("T, E, W, marked", [(1024, 64, 8, True), (2047, 64, 8, True), (2048, 64, 8, False),
+                                             (1024, 8, 8, False), (1024, 64, 64, True)])
+def test_weight_rows_marked_by_pairs_per_expert(T, E, W, marked):
+    from torch.profiler import ProfilerActivity, profile
+
+    moe = _moe()
+    H, I, topk = 256, 128, 4
+    x, tw, ids, *_ = _case(T, W, H, I, T, topk)
+    ids = np.random.default_rng(T).integers(0, E, (T, topk))
+    *_, w13, w13s, w2, w2s = _case(T, W, H, I, 1, 1)
+    xb, (tw_t, ids_t, *w) = _bf16(x), _dev(tw, ids, w13, w13s, w2, w2s)
+    emap = torch.full((E,), -1, dtype=torch.int32, device="cuda")
+    emap[:W] = torch.arange(W, dtype=torch.int32, device="cuda")
+    xq, xs = moe.quant_tokens(xb)
+    r = moe.route(ids_t, emap, W)
+    contrib = torch.empty((T * topk, H), dtype=torch.bfloat16, device="cuda")
+    calls = [lambda: moe.run_experts(xq, xs, tw_t, *w, r, contrib),
+             lambda: moe.fused_moe(xb, tw_t, ids_t, *w, expert_map=emap)]
+    for call in calls:
+        call()
+        torch.cuda.synchronize()
+        with profile(activities=[ProfilerActivity.CUDA]) as prof:
+            call()
+            torch.cuda.synchronize()
+        names = [e.name for e in prof.events() if "gemm1_kernel<" in e.name or "gemm2_kernel<" in e.name]
+        assert len(names) == 2
+        assert all(("true>" in n.split("(unsigned")[0].split("(long")[0]) == marked for n in names), names

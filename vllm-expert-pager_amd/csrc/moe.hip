@@ -629,11 +629,15 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t off, void* dst)
 // they should not push the activation rows (re-read by every column block of a
 // tile) out of the caches. Where experts have several tiles, each reads the
 // rows again, and marked rows are no longer in its L2: dma_weights<false>.
-// Whole layers of 2048 x 512 experts, marked and not: 23 tokens (4 layers) 287
-// and 305 us, 333 tokens 97 and 101, 2048 tokens (64 pairs per expert) 246 and
-// 244, 8192 tokens (256) 566 and 533. So the line is a mean of one whole tile
-// (stream_weights). Chosen per item, by a branch around the loads, it cost the
-// small calls 20%.
+// Whole layers of 256 experts 2048 x 512 at top-8, marked and not, by the mean
+// pairs per expert: 16 (512 tokens) 177 and 186 us, 64 251 and 248, 128 372 and
+// 346, 256 566 and 533. Through chunks of 64 of these experts 16 (512 tokens)
+// 245 and 255, 32 295 and 305, 64 406 and 403, 128 474 and 463; of 16 experts
+// 16 639 and 652, 32 793 and 803, 64 882 and 883. 23 tokens (4 layers) 287 and
+// 305, 333 tokens of 64 experts 97 and 101. So the line is a mean of one whole
+// tile per expert (stream_weights): of the experts that the pairs spread over,
+// not of the slots of the slab, which holds a chunk of them. Chosen per item,
+// by a branch around the loads, it cost the small calls 20%.
 __device__ __forceinline__ void dma16_stream(const void* base, uint32_t off, void* dst) {
   uint32_t saved;
   asm volatile(
@@ -649,7 +653,7 @@ __device__ __forceinline__ void dma_weights(const void* base, uint32_t off, void
   else
     dma16(base, off, dst);
 }
-inline bool stream_weights(int64_t npairs, int64_t slots) { return npairs < slots * kWM; }
+inline bool stream_weights(int64_t npairs, int64_t num_experts) { return npairs < num_experts * kWM; }
 __device__ __forceinline__ void dma4(const void* base, uint32_t off, void* dst) {
   uint32_t saved;
   asm volatile(
@@ -2202,10 +2206,11 @@ int cus_per_xcd(int* out) {
 
 // The two (or, for few pairs, narrow) GEMM launches of one expert call over a
 // workspace of xp_moe_workspace_bytes(T * topk, I) bytes at `work`.
+// num_experts: the experts that the T * topk pairs are spread over.
 int launch_experts(const uint8_t* xq, const float* xs, int64_t T, int64_t topk, const float* topk_weight, int64_t H,
                    int64_t I, const uint8_t* w13, const float* w13_scale, const uint8_t* w2, const float* w2_scale,
-                   int64_t slots, const int32_t* offsets, const int32_t* pairs, const int32_t* tiles, uint8_t* work,
-                   uint16_t* out, int act, void* stream) {
+                   int64_t slots, int64_t num_experts, const int32_t* offsets, const int32_t* pairs,
+                   const int32_t* tiles, uint8_t* work, uint16_t* out, int act, void* stream) {
   const int64_t npairs = T * topk;
   const int64_t bound = tile_bound(npairs, slots);
   Work w;
@@ -2229,7 +2234,7 @@ int launch_experts(const uint8_t* xq, const float* xs, int64_t T, int64_t topk, 
     const int64_t per_xcd_tiles = (wmax + 7) / 8;  // wide tiles of one XCD, at most
     // One workgroup per CU: the operand ring takes most of its LDS.
     const int64_t n1 = std::min<int64_t>(per_xcd, per_xcd_tiles * (I / (16 * kGemmWaves)));
-    const bool stream_w = stream_weights(npairs, slots);
+    const bool stream_w = stream_weights(npairs, num_experts);
     auto* gemm1 = act == XP_ACT_GELU
                       ? (stream_w ? gemm1_kernel<XP_ACT_GELU, true> : gemm1_kernel<XP_ACT_GELU, false>)
                       : (stream_w ? gemm1_kernel<XP_ACT_SILU, true> : gemm1_kernel<XP_ACT_SILU, false>);
@@ -2349,28 +2354,39 @@ int xp_moe_layer(const uint16_t* x, int64_t T, int64_t H, const void* topk_ids, 
   rc = launch_route(x, T, H, w.xq, w.xs, topk_ids, topk_elem_bytes, T * topk, expert_map, num_experts, slots,
                     w.offsets, w.pairs, w.tiles, stream);
   if (rc) return rc;
-  rc = launch_experts(w.xq, w.xs, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots, w.offsets,
-                      w.pairs, w.tiles, w.ffn, w.contrib, activation, stream);
+  rc = launch_experts(w.xq, w.xs, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots, num_experts,
+                      w.offsets, w.pairs, w.tiles, w.ffn, w.contrib, activation, stream);
   if (rc) return rc;
   // Without a map expert e has slot e, so the sum's bound on the ids says it all.
   const int64_t E = expert_map || num_experts < slots ? num_experts : slots;
   return launch_topk_sum(w.contrib, T, topk, H, topk_ids, topk_elem_bytes, E, expert_map, slots, out, stream);
 }
 
-int xp_moe_experts(const uint8_t* xq, const float* xs, int64_t T, int64_t topk, const float* topk_weight, int64_t H,
-                   int64_t I, const uint8_t* w13, const float* w13_scale, const uint8_t* w2, const float* w2_scale,
-                   int64_t slots, const int32_t* offsets, const int32_t* pairs, const int32_t* tiles, void* work,
-                   int64_t work_bytes, uint16_t* out, int activation, void* stream) {
+int xp_moe_experts_part(const uint8_t* xq, const float* xs, int64_t T, int64_t topk, const float* topk_weight,
+                        int64_t H, int64_t I, const uint8_t* w13, const float* w13_scale, const uint8_t* w2,
+                        const float* w2_scale, int64_t slots, int64_t num_experts, const int32_t* offsets,
+                        const int32_t* pairs, const int32_t* tiles, void* work, int64_t work_bytes, uint16_t* out,
+                        int activation, void* stream) {
   int rc = check_experts("xp_moe_experts", xq, xs, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots,
                          offsets, pairs, tiles, out, activation);
-  if (rc || T == 0) return rc;
+  if (rc) return rc;
+  XP_REQUIRE(num_experts >= 1 && num_experts <= INT32_MAX, "xp_moe_experts: %lld experts", (long long)num_experts);
+  if (T == 0) return XP_OK;
   XP_REQUIRE(work && (reinterpret_cast<uintptr_t>(work) & 255) == 0,
              "xp_moe_experts: the workspace must be non-null and 256-byte aligned");
   const int64_t need = xp_moe_workspace_bytes(T * topk, I);
   XP_REQUIRE(work_bytes >= need, "xp_moe_experts: workspace of %lld B, needs %lld", (long long)work_bytes,
              (long long)need);
-  return launch_experts(xq, xs, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots, offsets, pairs,
-                        tiles, static_cast<uint8_t*>(work), out, activation, stream);
+  return launch_experts(xq, xs, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots, num_experts, offsets,
+                        pairs, tiles, static_cast<uint8_t*>(work), out, activation, stream);
+}
+
+int xp_moe_experts(const uint8_t* xq, const float* xs, int64_t T, int64_t topk, const float* topk_weight, int64_t H,
+                   int64_t I, const uint8_t* w13, const float* w13_scale, const uint8_t* w2, const float* w2_scale,
+                   int64_t slots, const int32_t* offsets, const int32_t* pairs, const int32_t* tiles, void* work,
+                   int64_t work_bytes, uint16_t* out, int activation, void* stream) {
+  return xp_moe_experts_part(xq, xs, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots, slots, offsets,
+                             pairs, tiles, work, work_bytes, out, activation, stream);
 }
 
 int xp_moe_experts_noalloc(const uint8_t* xq, const float* xs, int64_t T, int64_t topk, const float* topk_weight,
@@ -2389,8 +2405,8 @@ int xp_moe_experts_noalloc(const uint8_t* xq, const float* xs, int64_t T, int64_
   uint8_t* work = nullptr;
   rc = moe_scratch_address(&work);
   if (rc) return rc;
-  return launch_experts(xq, xs, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots, offsets, pairs,
-                        tiles, work, out, activation, stream);
+  return launch_experts(xq, xs, T, topk, topk_weight, H, I, w13, w13_scale, w2, w2_scale, slots, slots, offsets,
+                        pairs, tiles, work, out, activation, stream);
 }
 
 int xp_moe_decode_experts(const uint16_t* x, int64_t T, int64_t H, const void* topk_ids, int topk_elem_bytes,

@@ -133,6 +133,7 @@ _SIGNATURES = {
     "xp_ssd_read_probe": (_I, [_I, _L, _P, _L, _I, _I, _P]),
     "xp_moe_decode_experts": (_I, [_P, _L, _L, _P, _I, _L, _P, _P, _P, _L, _L, _P, _P, _P, _P, _L, _P, _L, _P, _I,
                                    _P]),
+    "xp_moe_experts_part": (_I, [_P, _P, _L, _L, _P, _L, _L, _P, _P, _P, _P, _L, _L, _P, _P, _P, _P, _L, _P, _I, _P]),
     "xp_moe_experts_noalloc": (_I, [_P, _P, _L, _L, _P, _L, _L, _P, _P, _P, _P, _L, _P, _P, _P, _P, _I, _P]),
     "xp_moe_layer_bytes": (_L, [_L, _L, _L, _L, _L]),
     "xp_moe_layer": (_I, [_P, _L, _L, _P, _I, _L, _P, _P, _L, _L, _P, _P, _P, _P, _L, _P, _L, _P, _I, _P]),

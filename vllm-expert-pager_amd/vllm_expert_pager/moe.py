@@ -81,6 +81,7 @@ class Routing:
     offsets: torch.Tensor  # int32 (slots + 1,)
     pairs: torch.Tensor  # int32 (T * topk,)
     tiles: torch.Tensor  # int32 (1 + 2 * bound,)
+    experts: int = 0  # entries of the expert_map (0: as many as slots)
 
     @property
     def count(self) -> torch.Tensor:
@@ -112,6 +113,7 @@ def _routing(topk_ids: torch.Tensor, expert_map: torch.Tensor, slots: int, out: 
             torch.empty((max(n, 1),), dtype=torch.int32, device=dev),
             torch.empty((1 + 2 * max(bound, 1),), dtype=torch.int32, device=dev),
         )
+    out.experts = expert_map.numel()
     return out
 
 
@@ -203,11 +205,11 @@ def run_experts(
     nbytes = int(nat.lib().xp_moe_workspace_bytes(T * topk, I))
     work = torch.empty((max(nbytes, 1),), dtype=torch.uint8, device=xq.device)
     nat.call(
-        "xp_moe_experts", _fp8_ptr(xq, "xq"), _f32(xs, "xs").data_ptr(), T, topk, tw.data_ptr(), H, I,
+        "xp_moe_experts_part", _fp8_ptr(xq, "xq"), _f32(xs, "xs").data_ptr(), T, topk, tw.data_ptr(), H, I,
         _fp8_ptr(w13, "w13"), _f32(w13_scale, "w13_scale").data_ptr(), _fp8_ptr(w2, "w2"),
-        _f32(w2_scale, "w2_scale").data_ptr(), routing.slots, routing.offsets.data_ptr(),
-        routing.pairs.data_ptr(), routing.tiles.data_ptr(), work.data_ptr(), nbytes, contrib.data_ptr(), act,
-        nat.stream(),
+        _f32(w2_scale, "w2_scale").data_ptr(), routing.slots, routing.experts or routing.slots,
+        routing.offsets.data_ptr(), routing.pairs.data_ptr(), routing.tiles.data_ptr(), work.data_ptr(), nbytes,
+        contrib.data_ptr(), act, nat.stream(),
     )
 
 

@@ -602,3 +602,27 @@ def test_weight_rows_marked_by_pairs_per_expert(T, E, W, marked):
         names = [e.name for e in prof.events() if "gemm1_kernel<" in e.name or "gemm2_kernel<" in e.name]
         assert len(names) == 2
         assert all(("true>" in n.split("(unsigned")[0].split("(long")[0]) == marked for n in names), names
+
+
+# The wide tiles' split over the XCDs in runs: every tile count around whole
+# turns of 16 tiles and below one, each slot's contributions against the
+# narrow kernels' (calls of fewer than 64 possible tiles).
+@pytest.mark.parametrize("live", [1, 7, 8, 15, 16, 17, 24, 31, 33, 100])
+def test_every_tile_count_of_the_split(live):
+    moe = _moe()
+    T, E, H, I = 120, 128, 384, 256
+    x, tw, _, w13, w13s, w2, w2s = _case(live, E, H, I, T, 1)
+    slot = np.sort(np.random.default_rng(live).permutation(E)[:live])
+    ids = slot[np.arange(T) % live].reshape(T, 1)
+    xb, (tw_t, ids_t, *w) = _bf16(x), _dev(tw, ids, w13, w13s, w2, w2s)
+    emap = torch.arange(E, dtype=torch.int32, device="cuda")
+    xq, xs = moe.quant_tokens(xb)
+
+    def contributions(t):
+        c = torch.zeros((xb[t].shape[0], H), dtype=torch.bfloat16, device="cuda")
+        moe.run_experts(xq[t], xs[t], tw_t[t], *w, moe.route(ids_t[t], emap, E), c)
+        return c.view(torch.int16)
+
+    whole = contributions(slice(0, T))  # 2 + 120 possible tiles: the prefill kernels
+    parts = torch.cat([contributions(slice(i, i + 40)) for i in range(0, T, 40)])
+    assert torch.equal(whole, parts)

@@ -1,9 +1,16 @@
 """Which kernels an expert FFN call takes, by sizes alone (CPU, no kernel is launched)."""
 
+import math
+import os
+import shutil
+import subprocess
+
 import pytest
 import torch
 
 from vllm_expert_pager import moe
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "vllm-expert-pager_amd", "csrc")
 
 
 # (T, topk, H, I): steps in which the fused launches were measured to be faster
@@ -23,3 +30,58 @@ def test_decode_pays(T, topk, H, I, pays):
     assert moe.decode_pays(x, ids, I) == pays
     if pays:
         assert moe.decode_fits(x, ids, I)
+
+
+@pytest.fixture(scope="module")
+def tile_split(tmp_path_factory):
+    """shares(live, runs): the list indices that each of the 8 XCDs takes, as csrc/tile_split.h has it."""
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    d = tmp_path_factory.mktemp("split")
+    src, exe = d / "split.cpp", d / "split"
+    src.write_text("""#include <cstdio>
+#include "tile_split.h"
+int main() {
+  for (int live = 0; live <= 400; ++live)
+    for (int runs = 0; runs < 2; ++runs)
+      for (int x = 0; x < xp::kXcds; ++x) {
+        std::printf("%d %d", live, runs);
+        for (int t = 0; t < xp::xcd_tiles(live, x, runs); ++t) std::printf(" %d", xp::xcd_tile(live, x, t, runs));
+        std::printf("\\n");
+      }
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    shares = {}
+    for line in subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.splitlines():
+        live, runs, *tiles = map(int, line.split())
+        shares.setdefault((live, bool(runs)), []).append(tiles)
+    return lambda live, runs: shares[live, runs]
+
+
+def test_tile_split_takes_every_tile_once(tile_split):
+    for live in range(401):
+        for runs in (False, True):
+            shares = tile_split(live, runs)
+            assert sorted(sum(shares, [])) == list(range(live))
+            # the launch's workgroups are sized for ceil(live / 8) tiles an XCD
+            assert {len(s) for s in shares} <= {live // 8, -(-live // 8)}
+
+
+def test_tile_split_shares_falling_popularity_evenly(tile_split):
+    """Lists whose tiles get lighter from slot to slot, by e^2 in all (experts of one tile each,
+    popular ones first): no XCD is further above the mean than its places in a turn, 7 before the
+    middle, and its share of the last turn make it. Eighths of the list give one twice the mean."""
+    for live in range(96, 401, 5):
+        pairs = [math.exp(-2.0 * i / live) for i in range(live)]
+        load = {runs: [sum(pairs[i] for i in s) for s in tile_split(live, runs)] for runs in (False, True)}
+        mean = sum(pairs) / 8
+        assert max(load[True]) < math.exp(14 / live) * math.ceil(live / 8) / (live / 8) * mean
+        assert max(load[False]) > 1.9 * mean
+
+
+def test_tile_split_keeps_an_experts_tiles_together(tile_split):
+    """Eighths: the tiles of an expert, neighbours in the list, are on one XCD but at 7 borders."""
+    for live in (8, 100, 399):
+        owner = {t: x for x, s in enumerate(tile_split(live, False)) for t in s}
+        assert sum(owner[t] != owner[t + 1] for t in range(live - 1)) == 7

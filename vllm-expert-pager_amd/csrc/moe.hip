@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "tile_split.h"
 
 namespace xp {
 namespace {
@@ -535,13 +536,12 @@ constexpr int kMaxKB = 64;    // K blocks a workgroup keeps row scales for (H, I
 
 // ---- prefill GEMMs: persistent workgroups over wide tiles ----
 //
-// A work item is (wide tile, column block). XCD x takes the x-th eighth of
-// the wide-tile list, a tile's column blocks consecutive; workgroup b runs on
-// XCD b % 8 and takes that XCD's items l, l + nl, l + 2 nl, ... (l = b / 8,
-// nl = gridDim.x / 8), so a tile's column blocks run side by side on one XCD
-// and its token rows are read into one L2, and the tiles of an expert with
-// more than kWM pairs, neighbours in the list, read its weight rows into one
-// L2 at about the same time.
+// A work item is (wide tile, column block). Every XCD takes its share of the
+// wide-tile list (tile_split.h), a tile's column blocks consecutive; workgroup
+// b runs on XCD b % 8 and takes that XCD's items l, l + nl, l + 2 nl, ... (l =
+// b / 8, nl = gridDim.x / 8), so a tile's column blocks run side by side on one
+// XCD and its token rows are read into one L2, and the tiles of an expert with
+// more than kWM pairs read its weight rows into one L2 at about the same time.
 //
 // The weight rows are the MFMA's A operand and the token rows its B operand,
 // so a lane's four outputs are four columns of one token row: one scale read
@@ -704,21 +704,21 @@ struct Item {
   int slot, first, count, col;  // count 0: no item
 };
 
-// Candidate n of this workgroup: item j = l + n * nl of its XCD, i.e. wide
-// tile base + j / ncols of the XCD's range and column block j % ncols. Its
+// Candidate n of this workgroup: item j = l + n * nl of its XCD, i.e. the
+// XCD's wide tile j / ncols (see tile_split.h) and column block j % ncols. Its
 // list entry is read through the scalar cache (the list does not change
 // during the call).
+template <bool RUNS>
 __device__ __forceinline__ Item item_fetch(int n, int ncols, const int32_t* __restrict__ wide, int64_t wmax) {
   const int jj = (static_cast<int>(blockIdx.x) >> 3) + n * (static_cast<int>(gridDim.x) >> 3);
   const int xcd = static_cast<int>(blockIdx.x) & 7;
   const int live = wide[0] < wmax ? wide[0] : static_cast<int>(wmax);
-  const int each = live >> 3, extra = live & 7;  // the first `extra` XCDs take one tile more
-  const int base = xcd * each + (xcd < extra ? xcd : extra);
-  const int w = __builtin_amdgcn_readfirstlane(base + jj / ncols);
+  const int t = jj / ncols;
   Item it;
-  it.col = __builtin_amdgcn_readfirstlane(jj - (jj / ncols) * ncols);
+  it.col = __builtin_amdgcn_readfirstlane(jj - t * ncols);
   it.slot = it.first = it.count = 0;
-  if (w < base + each + (xcd < extra ? 1 : 0)) {
+  if (t < xcd_tiles(live, xcd, RUNS)) {
+    const int w = __builtin_amdgcn_readfirstlane(xcd_tile(live, xcd, t, RUNS));
     it.slot = wide[1 + 3 * static_cast<int64_t>(w)];
     it.first = wide[2 + 3 * static_cast<int64_t>(w)];
     it.count = wide[3 + 3 * static_cast<int64_t>(w)];
@@ -796,9 +796,9 @@ __global__ void __launch_bounds__(kGemmWaves * 64) gemm1_kernel(const uint8_t* _
   const int q = lane >> 4, j = lane & 15;
   const int KB = static_cast<int>(H / kKB), KS = KB > kMinSteps ? KB : kMinSteps;
 
-  Item cur = item_fetch(0, ncols, wide, wmax);
+  Item cur = item_fetch<STREAM>(0, ncols, wide, wmax);
   if (cur.count == 0) return;
-  Item nxt = item_fetch(1, ncols, wide, wmax);
+  Item nxt = item_fetch<STREAM>(1, ncols, wide, wmax);
   int n = 2;
 
   // Weight-row loads: load i of a wave covers its stage rows 8i .. 8i + 7,
@@ -897,7 +897,7 @@ __global__ void __launch_bounds__(kGemmWaves * 64) gemm1_kernel(const uint8_t* _
         if (more) {
           if (k == 0) {
             request_pairs(nxt, pairs, s_pn);
-            after = item_fetch(n, ncols, wide, wmax);
+            after = item_fetch<STREAM>(n, ncols, wide, wmax);
           } else if (k == 1) {
             put_rows(nxt, s_pn, topk, npairs, s_pair[nb], s_row[nb]);
           } else if (k == 2) {
@@ -1829,9 +1829,9 @@ __global__ void __launch_bounds__(kGemmWaves * 64) gemm2_kernel(int64_t H, int64
   const int q = lane >> 4, j = lane & 15;
   const int KB = static_cast<int>(I / kKB), KS = KB > kMinSteps ? KB : kMinSteps;
 
-  Item cur = item_fetch(0, ncols, wide, wmax);
+  Item cur = item_fetch<STREAM>(0, ncols, wide, wmax);
   if (cur.count == 0) return;
-  Item nxt = item_fetch(1, ncols, wide, wmax);
+  Item nxt = item_fetch<STREAM>(1, ncols, wide, wmax);
   int n = 2;
 
   // Weight-row loads: load i of a wave covers its stage rows 8i .. 8i + 7,
@@ -1924,7 +1924,7 @@ __global__ void __launch_bounds__(kGemmWaves * 64) gemm2_kernel(int64_t H, int64
         if (more) {
           if (k == 0) {
             request_pairs(nxt, pairs, s_pn);
-            after = item_fetch(n, ncols, wide, wmax);
+            after = item_fetch<STREAM>(n, ncols, wide, wmax);
           } else if (k == 1) {
             put_rows(nxt, s_pn, 1, npairs, s_pair[nb], s_row[nb]);
           } else if (k == 2) {

@@ -915,7 +915,7 @@ int xp_encode_rows_split(const uint8_t* raw, int64_t rows, int64_t raw_stride, i
     hipLaunchKernelGGL(encode_count_kernel, plan_grid, dim3(kThreads), 0, as_stream(stream), a);
   else
     hipLaunchKernelGGL(encode_hist_kernel, plan_grid, dim3(kThreads), 0, as_stream(stream), a);
-  if (int rc = check_launch("encode_hist_kernel")) return rc;
+  if (int rc = check_launch(counted ? "encode_count_kernel" : "encode_hist_kernel")) return rc;
   // Counted chunks: a workgroup's threads take 8 groups at once.
   int64_t groups = counted ? kGroupsPerBlock : 1;
   while (groups < (counted ? kMaxGroups : kGroupsPerBlock) && rows * ((G + groups - 1) / groups) > kWordsBlocks)
@@ -930,7 +930,7 @@ int xp_encode_rows_split(const uint8_t* raw, int64_t rows, int64_t raw_stride, i
   else
     hipLaunchKernelGGL(encode_words_kernel, words_grid, dim3(kThreads), 0, as_stream(stream), a,
                        static_cast<int>(groups), static_cast<int>(word_blocks));
-  if (int rc = check_launch("encode_words_kernel")) return rc;
+  if (int rc = check_launch(counted ? "encode_sizes_kernel" : "encode_words_kernel")) return rc;
   if (rows * G <= kSegmentGroups && chunk >= kSegments * kMinSegment) {
     const int64_t pairs = (G + 1) / 2;
     hipLaunchKernelGGL((encode_groups_kernel<true, kSegments>), dim3(static_cast<unsigned>(rows * pairs)),

@@ -3,7 +3,9 @@
 // (codec_host.cpp) and of the reference.
 //
 // The plan: encode_hist_kernel and encode_words_kernel (chunks of 512 values
-// and more: encode_count_kernel and encode_sizes_kernel), several workgroups per row, or without a workspace encode_plan_kernel, one per row:
+// and more: encode_count_kernel and encode_sizes_kernel), several workgroups
+// per row; or encode_plan_kernel, one per row, for C callers of xp_encode_rows,
+// which has no workspace (the Python package always gives one):
 //   1. exponent histogram: per-thread counters in LDS, then summed;
 //   2. the code by one wave, the 512-entry LUT by the workgroup;
 //   3. Huffman words per chunk: the decoder loads a word before symbol i
@@ -206,8 +208,8 @@ __device__ __forceinline__ void write_lut(const int32_t* s_len, const int32_t* s
 // With a workspace the plan's two passes are launches of their own over
 // parts of the rows, so that a few rows fill the GPU and many rows leave no
 // partly empty round of one workgroup per row. One 2 MiB row: 266 us in one
-// workgroup, 7 + 12 us here; 256 rows: 316 us, 111 + 142 us (537 MB read
-// twice, at 4.8 and 3.8 TB/s; half of what was saved is the code's). Long
+// workgroup, 7 + 12 us here; 256 rows: 316 us, 119 + 143 us (537 MB read
+// twice, at 4.5 and 3.8 TB/s; half of what was saved is the code's). Long
 // chunks are read once, see encode_count_kernel.
 
 // Exponent counts of part `blockIdx.x % parts` (kPartBytes values) of a row.
@@ -433,7 +435,7 @@ __global__ void __launch_bounds__(kThreads) encode_sizes_kernel(EncodeArgs a, in
   }
 }
 
-// ---- the plan of a row by one workgroup ----
+// ---- the plan of a row by one workgroup: xp_encode_rows ----
 __global__ void __launch_bounds__(kPlanThreads) encode_plan_kernel(EncodeArgs a) {
   __shared__ uint32_t s_hist[code::kSyms][kPlanThreads];  // per-thread counters
   __shared__ int32_t s_len[code::kSyms];

@@ -137,12 +137,15 @@ def test_encode_of_a_gpu_row():
 
 # The plan by several workgroups per row against the one by a workgroup per
 # row: rows of 1, 2, 4 and 8 groups per counting workgroup (up to 2048
-# workgroups take one group each), more than one 64 KiB part per row, chunks that
-# are counted (from 512 values, with a partial last part and more groups than a
-# workgroup takes at once), and rows
-# that do not fit, whose records stay as they were.
+# workgroups take one group each), more than one 64 KiB part per row, chunks
+# that are counted (from 512 values, with a partial last part), counted rows
+# whose workgroups take 16 groups, 8 at once (above 2048 workgroups of 8 groups:
+# 1500 rows of 9 groups, 700 of 17) and whose groups fill the chip unsegmented
+# with a spare half-wave, and rows that do not fit, whose records stay as they
+# were.
 @pytest.mark.parametrize("count, groups, chunk", [(1, 1, 16), (1, 130, 64), (300, 9, 16), (700, 11, 16),
-                                                  (1500, 17, 16), (3, 40, 1024), (2, 5, 512), (300, 9, 512), (5, 9, 1024)])
+                                                  (1500, 17, 16), (3, 40, 1024), (2, 5, 512), (300, 9, 512),
+                                                  (5, 9, 1024), (1500, 9, 512), (700, 17, 512)])
 def test_split_plan_equals_a_workgroup_per_row(count, groups, chunk):
     from vllm_expert_pager import _native as nat
 

@@ -118,8 +118,6 @@ def test_quant_tokens_bit_exact():
     assert np.array_equal(xs.cpu().numpy(), s)
 
 
-# 5000 x 8 pairs: each of the 16 waves walks 2500 pairs, in batches of 1024
-# (the last one partial).
 def test_quant_tokens_of_every_maximum():
     """Groups whose maxima are all the finite bf16 magnitudes, their other values spread
     below (signed zeros and subnormals among them), give the codes of a division by the
@@ -148,6 +146,8 @@ def test_quant_tokens_of_every_maximum():
     np.testing.assert_array_equal(code[:, 2:], np.where(sign, 0x80, 0))
 
 
+# 5000 x 8 pairs: counted and scattered by 40 workgroups of 1000 pairs; the
+# others by one workgroup, whose 16 waves take at most 256 pairs each.
 @pytest.mark.parametrize("T, topk, E, slots", [(50, 4, 20, 12), (300, 4, 6, 6), (1, 8, 64, 32), (5000, 8, 256, 200)])
 def test_route_lists_mapped_pairs(T, topk, E, slots):
     moe = _moe()

@@ -604,9 +604,9 @@ def test_weight_rows_marked_by_pairs_per_expert(T, E, W, marked):
         assert all(("true>" in n.split("(unsigned")[0].split("(long")[0]) == marked for n in names), names
 
 
-# The wide tiles' split over the XCDs in runs: every tile count around whole
-# turns of 16 tiles and below one, each slot's contributions against the
-# narrow kernels' (calls of fewer than 64 possible tiles).
+# The wide tiles' split over the XCDs in halves: tile counts around multiples of
+# 16 and below, each slot's contributions against the narrow kernels' (calls of
+# fewer than 64 possible tiles).
 @pytest.mark.parametrize("live", [1, 7, 8, 15, 16, 17, 24, 31, 33, 100])
 def test_every_tile_count_of_the_split(live):
     moe = _moe()

@@ -34,7 +34,7 @@ def test_decode_pays(T, topk, H, I, pays):
 
 @pytest.fixture(scope="module")
 def tile_split(tmp_path_factory):
-    """shares(live, runs): the list indices that each of the 8 XCDs takes, as csrc/tile_split.h has it."""
+    """shares(live, halves): the list indices that each of the 8 XCDs takes, as csrc/tile_split.h has it."""
     if shutil.which("g++") is None:
         pytest.skip("no g++")
     d = tmp_path_factory.mktemp("split")
@@ -43,10 +43,10 @@ def tile_split(tmp_path_factory):
 #include "tile_split.h"
 int main() {
   for (int live = 0; live <= 400; ++live)
-    for (int runs = 0; runs < 2; ++runs)
-      for (int x = 0; x < xp::kXcds; ++x) {
-        std::printf("%d %d", live, runs);
-        for (int t = 0; t < xp::xcd_tiles(live, x, runs); ++t) std::printf(" %d", xp::xcd_tile(live, x, t, runs));
+    for (int halves = 0; halves < 2; ++halves)
+      for (int x = 0; x < 8; ++x) {
+        std::printf("%d %d", live, halves);
+        for (int t = 0; t <= live / 8 + 2; ++t) std::printf(" %d", xp::xcd_tile(live, x, t, halves));
         std::printf("\\n");
       }
 }
@@ -54,34 +54,38 @@ int main() {
     subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(src), "-o", str(exe)], check=True)
     shares = {}
     for line in subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.splitlines():
-        live, runs, *tiles = map(int, line.split())
-        shares.setdefault((live, bool(runs)), []).append(tiles)
-    return lambda live, runs: shares[live, runs]
+        live, halves, *tiles = map(int, line.split())
+        n = sum(w < live for w in tiles)
+        # workgroups stop at the first tile that is not there
+        assert all(0 <= w < live for w in tiles[:n]) and min(tiles[n:]) >= live
+        shares.setdefault((live, bool(halves)), []).append(tiles[:n])
+    return lambda live, halves: shares[live, halves]
 
 
 def test_tile_split_takes_every_tile_once(tile_split):
     for live in range(401):
-        for runs in (False, True):
-            shares = tile_split(live, runs)
+        for halves in (False, True):
+            shares = tile_split(live, halves)
             assert sorted(sum(shares, [])) == list(range(live))
             # the launch's workgroups are sized for ceil(live / 8) tiles an XCD
             assert {len(s) for s in shares} <= {live // 8, -(-live // 8)}
 
 
-def test_tile_split_shares_falling_popularity_evenly(tile_split):
+def test_tile_split_shares_falling_popularity(tile_split):
     """Lists whose tiles get lighter from slot to slot, by e^2 in all (experts of one tile each,
-    popular ones first): no XCD is further above the mean than its places in a turn, 7 before the
-    middle, and its share of the last turn make it. Eighths of the list give one twice the mean."""
+    popular ones first). Halves: an XCD has two sixteenths, places p and 15 - p of 16, so the most
+    is cosh(15/16) / cosh(1/16) of the least, 1.26 of the mean and a tile of the last 15 more.
+    Eighths of the list give one XCD twice the mean."""
     for live in range(96, 401, 5):
         pairs = [math.exp(-2.0 * i / live) for i in range(live)]
-        load = {runs: [sum(pairs[i] for i in s) for s in tile_split(live, runs)] for runs in (False, True)}
+        load = {halves: [sum(pairs[i] for i in s) for s in tile_split(live, halves)] for halves in (False, True)}
         mean = sum(pairs) / 8
-        assert max(load[True]) < math.exp(14 / live) * math.ceil(live / 8) / (live / 8) * mean
+        assert max(load[True]) < 1.26 * mean + pairs[live // 16 * 16 - 1]
         assert max(load[False]) > 1.9 * mean
 
 
 def test_tile_split_keeps_an_experts_tiles_together(tile_split):
-    """Eighths: the tiles of an expert, neighbours in the list, are on one XCD but at 7 borders."""
+    """The tiles of an expert, neighbours in the list, are on one XCD but at 7 borders of eighths."""
     for live in (8, 100, 399):
         owner = {t: x for x, s in enumerate(tile_split(live, False)) for t in s}
         assert sum(owner[t] != owner[t + 1] for t in range(live - 1)) == 7

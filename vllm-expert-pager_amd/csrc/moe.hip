@@ -708,17 +708,16 @@ struct Item {
 // XCD's wide tile j / ncols (see tile_split.h) and column block j % ncols. Its
 // list entry is read through the scalar cache (the list does not change
 // during the call).
-template <bool RUNS>
+template <bool HALVES>
 __device__ __forceinline__ Item item_fetch(int n, int ncols, const int32_t* __restrict__ wide, int64_t wmax) {
   const int jj = (static_cast<int>(blockIdx.x) >> 3) + n * (static_cast<int>(gridDim.x) >> 3);
-  const int xcd = static_cast<int>(blockIdx.x) & 7;
   const int live = wide[0] < wmax ? wide[0] : static_cast<int>(wmax);
   const int t = jj / ncols;
+  const int w = __builtin_amdgcn_readfirstlane(xcd_tile(live, static_cast<int>(blockIdx.x) & 7, t, HALVES));
   Item it;
   it.col = __builtin_amdgcn_readfirstlane(jj - t * ncols);
   it.slot = it.first = it.count = 0;
-  if (t < xcd_tiles(live, xcd, RUNS)) {
-    const int w = __builtin_amdgcn_readfirstlane(xcd_tile(live, xcd, t, RUNS));
+  if (w < live) {
     it.slot = wide[1 + 3 * static_cast<int64_t>(w)];
     it.first = wide[2 + 3 * static_cast<int64_t>(w)];
     it.count = wide[3 + 3 * static_cast<int64_t>(w)];

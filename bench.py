@@ -331,7 +331,7 @@ def bench_encode(args, dev, cores):
     cpu_gbps = n_cpu * sum(r.shape[1] for r in raws) / cpu_s / 1e9
     out = {
         "workload": f"encode {count} experts (w13 fp8 1024x2048 + w2 fp8 2048x512 rows, block-scaled N(0,0.02)) "
-                    "at pitch 0.89, one launch per name",
+                    "at pitch 0.89, one call per name",
         "ms": round(ms, 4),
         "raw_gbps": round(raw_bytes / (ms * 1e-3) / 1e9, 2),
         "hbm_gbps": round((raw_bytes + out_bytes) / (ms * 1e-3) / 1e9, 2),

@@ -304,7 +304,8 @@ int xp_encode_row(const uint8_t* raw, int64_t n, int64_t chunk,
  * bytes xp_encode_row writes. needed[r] (device) receives each record's used
  * bytes; a row whose needed[r] exceeds pitch writes only its LUT, and the
  * caller reports it as xp_encode_row's XP_E_PITCH. All pointers are device
- * memory; enqueued on `stream`.
+ * memory; two launches on `stream`, one workgroup planning a row
+ * (xp_encode_rows_split is faster, for a workspace).
  * Replaces encode (codec.py:125-198), called per row at load time
  * (store.py:588). */
 int xp_encode_rows(const uint8_t* raw, int64_t rows, int64_t raw_stride,
@@ -488,7 +489,7 @@ int xp_moe_experts_noalloc(const uint8_t* xq, const float* xs, int64_t T,
  * xp_moe_quant_route + xp_moe_experts + xp_moe_topk_sum, but the routing and
  * quantisation run inside the gate/up launch and each token's top-k sum
  * inside the down-projection launch (one workgroup per token and 8
- * columns). Replaces, like those calls, fused_experts + moe_sum of a step
+ * columns, 16 from two tokens on). Replaces, like those calls, fused_experts + moe_sum of a step
  * whose experts are all in the slab (experts.py:579-604): every pair with a
  * valid id should have a slot (one without adds nothing here). work is
  * xp_moe_workspace_bytes(T * topk, I) bytes, 256-byte aligned. Fails with

@@ -6,7 +6,7 @@ intercepts ``moe_sum`` to take the top-k sum once over all chunks
 (experts.py:538-556). Weights are w8a8 block-fp8: e4m3 rows with one fp32
 scale per 128x128 block, activations quantised per token and 128 columns.
 
-The work of one MoE call is split in four launches so that the overflow path
+The work of one MoE call is split in four calls so that the overflow path
 can quantise once, run the experts chunk by chunk, and combine once:
 
     xq, xs = quant_tokens(x)
@@ -131,7 +131,7 @@ def route(topk_ids: torch.Tensor, expert_map: torch.Tensor, slots: int, out: Rou
 
 def quant_route(x: torch.Tensor, topk_ids: torch.Tensor, expert_map: torch.Tensor,
                 slots: int) -> tuple[torch.Tensor, torch.Tensor, Routing]:
-    """``quant_tokens(x)`` and ``route(topk_ids, expert_map, slots)`` in one launch."""
+    """``quant_tokens(x)`` and ``route(topk_ids, expert_map, slots)`` in one launch (two above 4096 pairs)."""
     nat.require_device(x, "x")
     if x.dtype != torch.bfloat16 or x.dim() != 2:
         raise ValueError(f"x must be a 2-D bfloat16 tensor, got {x.dtype} {tuple(x.shape)}")

@@ -418,7 +418,7 @@ class Store:
 
         ``rows`` is ``(n, row_bytes)`` of any 1-byte dtype on any device.
         Compressed tiers encode the rows on the GPU when they are there
-        (one launch for all of them), else in a thread pool (the host
+        (one call for all of them), else in a thread pool (the host
         encoder releases the GIL); RAM-tier slots 0..min(n, R)-1 of the layer
         are filled with one copy and each expert's record goes to the paging
         file.
